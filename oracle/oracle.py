@@ -44,7 +44,8 @@ def build() -> None:
     """Compile liboracle.so (and the reference host functions when the
     reference tree is present)."""
     subprocess.check_call(["make", "-s", "-B", "-C", HERE, "liboracle.so"])
-    if os.path.isdir(os.environ.get("SBLAS_REFERENCE_DIR", "/root/reference")):
+    ref = os.environ.get("SBLAS_REFERENCE_DIR", "/root/reference")
+    if os.path.exists(os.path.join(ref, "src", "spmv_helper.cu")):
         subprocess.check_call(["sh", os.path.join(HERE, "build_ref.sh")],
                               stdout=subprocess.DEVNULL)
 
