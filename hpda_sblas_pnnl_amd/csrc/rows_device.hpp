@@ -1,12 +1,23 @@
-// rows_device.hpp -- the row sums of an LDS-staged row block, shared by the
-// row-block kernel (sblas_vector.hip) and the column-sorted row blocks
-// (sblas_sorted.hip).
+// rows_device.hpp -- what the row-block kernels share: the block order over the
+// XCDs (sblas_vector.hip, sblas_spmm.hip) and the row sums of an LDS-staged row
+// block (sblas_vector.hip, the column-sorted row blocks in sblas_sorted.hip).
 #pragma once
 
 #include "internal.hpp"
 
 namespace sblas {
 namespace rows {
+
+// The block this workgroup takes, -1 for none.  With xcd_remap (grid a
+// multiple of 8) each XCD takes a contiguous eighth of the blocks.
+__device__ __forceinline__ int logical_block(int total_blocks, int xcd_remap) {
+  int b = blockIdx.x;
+  if (xcd_remap) {
+    const int per = gridDim.x >> 3;
+    b = (b & 7) * per + (b >> 3);
+  }
+  return b < total_blocks ? b : -1;
+}
 
 // Sum over the W lanes of each aligned group of W lanes (xor butterfly).
 template <int W>

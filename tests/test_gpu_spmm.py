@@ -1,0 +1,80 @@
+"""Multi-vector products over row blocks (csrc/sblas_spmm.hip) against the
+FP64 oracle, at the sizes where spans, row ends and block edges meet.
+
+Bound: two sums of a row's L products in different orders, each off by at most
+(L + 3) roundings of 2^-53 of alpha * sum |a x| + |beta y| (the products, the
+additions, the scaling by alpha and the add of beta*y), so their difference by
+twice that.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+EPS = 2.0 ** -53
+DTYPES = ["f64", "f32", "bf16"]
+
+
+def _rows(lens, n, rng):
+    rp = np.zeros(len(lens) + 1, np.int64)
+    np.cumsum(lens, out=rp[1:])
+    col = np.concatenate([np.sort(rng.choice(n, size=k, replace=False)) for k in lens if k]
+                         or [np.zeros(0, np.int64)])
+    return rp.astype(np.int32), col.astype(np.int32)
+
+
+# row lengths: one element a row; spans of eight and blocks of 2048 met exactly
+# and by one; rows of a block's size and across blocks; the row limit of a block
+# with empty rows at its ends; nothing at all
+SHAPES = {
+    "ones": [1] * 2500,
+    "eights": [8] * 700,
+    "sevens_nines": [7, 9] * 400,
+    "block_edges": [2047, 1, 2048, 2049, 1, 4096, 3, 5000],
+    "empty_ends": [0] * 1023 + [5] + [0] * 1100 + [1, 0, 2] * 300 + [0] * 70,
+    "ragged": [int(v) for v in np.random.default_rng(3).geometric(0.06, 900)],
+    "short_block": [3, 0, 4, 65],
+    "empty": [0] * 40,
+}
+
+
+@pytest.mark.parametrize("shape", list(SHAPES))
+@pytest.mark.parametrize("k", [2, 4, 8, 16])
+def test_spmm_blocks(oracle, shape, k):
+    import torch
+    from hpda_sblas_pnnl_amd import gen as G
+    from hpda_sblas_pnnl_amd.device import SpmvPlan
+    rng = np.random.default_rng(17 * k + len(shape))
+    lens, n = SHAPES[shape], 6000
+    m = len(lens)
+    rp, col = _rows(lens, n, rng)
+    wide = rng.standard_normal(len(col))
+    dtype = DTYPES[(k + len(shape)) % 3]
+    if dtype == "f64":
+        val, dval = wide, torch.from_numpy(wide).cuda()
+    elif dtype == "f32":
+        val = wide.astype(np.float32).astype(np.float64)
+        dval = torch.from_numpy(wide.astype(np.float32)).cuda()
+    else:
+        bits = G.to_bf16_bits(wide)
+        val = G.from_bf16_bits(bits)
+        dval = torch.from_numpy(bits.view(np.int16)).cuda()
+    X, Y0 = rng.uniform(-1, 1, (n, k)), rng.uniform(-1, 1, (m, k))
+    absx = oracle.csr_spmm(m, k, np.abs(val), rp, col, np.abs(X), 1.0, 0.0, np.zeros((m, k)))
+    # X and Y start 8 bytes past a 16-byte boundary
+    dX = torch.empty(n * k + 1, dtype=torch.float64, device="cuda")[1:].view(n, k)
+    dX.copy_(torch.from_numpy(X))
+    drp, dcol = torch.from_numpy(rp).cuda(), torch.from_numpy(col).cuda()
+    for chunks, items in ((1, 0), (3, 16)):
+        plan = SpmvPlan("csr", m, n, drp, dcol, dval, kernel="vector", variant=2, chunks=chunks,
+                        items=items)
+        for alpha, beta in ((1.0, 0.0), (-0.75, 0.5)):
+            buf = torch.full((m * k + 3,), 7.0, dtype=torch.float64, device="cuda")
+            dY = buf[1:m * k + 1].view(m, k)
+            dY.copy_(torch.from_numpy(Y0))
+            plan.spmm(dX, dY, alpha, beta)
+            ref = oracle.csr_spmm(m, k, val, rp, col, X, alpha, beta, Y0).reshape(m, k)
+            scale = abs(alpha) * absx.reshape(m, k) + abs(beta) * np.abs(Y0)
+            bound = 2 * (np.asarray(lens)[:, None] + 3) * EPS * scale
+            assert (np.abs(dY.cpu().numpy() - ref) <= bound).all()
+            assert buf[0] == 7.0 and (buf[m * k + 1:] == 7.0).all()
