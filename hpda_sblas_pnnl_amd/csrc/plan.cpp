@@ -92,8 +92,9 @@ namespace {
 
 // Cached decisions of the timed trial, keyed by the row-length profile.
 struct TuneKey {
-  int val_type, mean_q, cv_q, empty_q, nnz_q;
+  int val_type, narrow_x, mean_q, cv_q, empty_q, nnz_q;
   bool operator<(const TuneKey &o) const {
+    if (narrow_x != o.narrow_x) return narrow_x < o.narrow_x;
     if (val_type != o.val_type) return val_type < o.val_type;
     if (mean_q != o.mean_q) return mean_q < o.mean_q;
     if (cv_q != o.cv_q) return cv_q < o.cv_q;
@@ -103,17 +104,22 @@ struct TuneKey {
 };
 struct TuneResult {
   int kernel, variant;
+  bool rows_x32;  // narrow values: row blocks gather x from an FP32 copy
   float ms[4];  // trial medians: row blocks, CSR5-style, column-sorted row blocks, segments
 };
 std::mutex g_tune_mu;
 std::map<TuneKey, TuneResult> g_tune_cache;
 
-TuneKey tune_key(int val_type, const RowStats &s, int64_t nnz) {
+TuneKey tune_key(int val_type, int narrow_x, const RowStats &s, int64_t nnz) {
   auto q = [](double v, double per_octave) {
     return static_cast<int>(std::lround(std::log2(std::max(v, 1e-3)) * per_octave));
   };
-  return TuneKey{val_type, q(s.mean, 4), q(1.0 + s.cv, 4),
-                 static_cast<int>(std::lround(s.empty_frac * 10)), q(static_cast<double>(nnz), 1)};
+  return TuneKey{val_type,
+                 narrow_x,
+                 q(s.mean, 4),
+                 q(1.0 + s.cv, 4),
+                 static_cast<int>(std::lround(s.empty_frac * 10)),
+                 q(static_cast<double>(nnz), 1)};
 }
 
 }  // namespace
@@ -828,6 +834,11 @@ int Plan::trial(const std::vector<std::pair<int, int>> &forms, std::vector<float
   return SBLAS_OK;
 }
 
+// opts.narrow_x, with SBLAS_NARROW_X in the place of the auto setting (0)
+int Plan::narrow_x_asked() const {
+  return opts.narrow_x != 0 ? opts.narrow_x : std::max(env_int("SBLAS_NARROW_X", 0), 0);
+}
+
 // Kernel choice and launch set-up for a CSR matrix whose row pointer is h_rp
 // (the caller's CSR, or the row-major form built from a CSC matrix).
 //
@@ -836,9 +847,9 @@ int Plan::trial(const std::vector<std::pair<int, int>> &forms, std::vector<float
 // pays for it (a structural test over the per-panel column ranges, measured
 // crossover; slices in row order for FP64 values, in sorted groups where x
 // is staged in FP32); otherwise the row-block form of kernel 1, its
-// column-sorted variant or the CSR5-style kernel 3 (tile depth sigma from the
-// reference's rule), whichever a timed trial on this matrix finds fastest.
-// Trials run for matrices of at least
+// column-sorted variant, row blocks over column segments or the CSR5-style
+// kernel 3 (tile depth sigma from the reference's rule), whichever a timed
+// trial on this matrix finds fastest.  Trials run for matrices of at least
 // 2^20 elements (smaller ones take row blocks) and are cached by row profile
 // (value type, mean, coefficient of variation, empty-row fraction, size),
 // so later plans of the same profile reuse the decision without a trial.
@@ -853,11 +864,8 @@ int Plan::finish_csr(const std::vector<int> &h_rp) {
   // BF16 values 1.14x -> 1.22x, normwise error 2.2e-8.  Auto leaves matrices
   // under 2^20 elements in FP64 x: their product is mostly launch latency,
   // and the copy's own launch made the power-law n = 2e4 matrix 0.70x.
-  int nxo = opts.narrow_x;
-  if (nxo == 0) {
-    nxo = env_int("SBLAS_NARROW_X", 0);
-    if (nxo <= 0) nxo = nnz >= (int64_t{1} << 20) ? 2 : 1;
-  }
+  int nxo = narrow_x_asked();
+  if (nxo == 0) nxo = nnz >= (int64_t{1} << 20) && rows_x32 ? 2 : 1;
   if ((variant == 2 || variant == 6) && kernel == SBLAS_KERNEL_VECTOR &&
       val_type != SBLAS_VAL_F64 && nxo == 2 && n > 0) {
     x32_rows = static_cast<float *>(dev_alloc(sizeof(float) * static_cast<size_t>(n)));
@@ -983,7 +991,8 @@ int Plan::choose_csr(const std::vector<int> &h_rp) {
   // the CSR5-style form
   if (!auto_kernel || opts.variant != 0 || opts.streams > 1 || nnz < (int64_t{1} << 20))
     return SBLAS_OK;
-  const TuneKey key = tune_key(val_type, stats, nnz);
+  const int narrow = narrow_x_asked();
+  const TuneKey key = tune_key(val_type, narrow, stats, nnz);
   TuneResult found{};
   bool cached = false;
   {
@@ -996,6 +1005,7 @@ int Plan::choose_csr(const std::vector<int> &h_rp) {
   }
   if (cached) {
     tuned = 3;
+    rows_x32 = found.rows_x32;
     for (int i = 0; i < 4; i++) trial_ms[i] = found.ms[i];
     if (found.kernel == SBLAS_KERNEL_CSR5) {
       kernel = SBLAS_KERNEL_CSR5;
@@ -1026,10 +1036,12 @@ int Plan::choose_csr(const std::vector<int> &h_rp) {
   if ((st = setup_csr5(h_rp)) != SBLAS_OK) return st;
   std::vector<std::pair<int, int>> forms{
       {SBLAS_KERNEL_VECTOR, 2}, {SBLAS_KERNEL_CSR5, 2}, {SBLAS_KERNEL_VECTOR, 4}};
-  // column segments where x is several times an XCD's L2 (4 MB), unless the
+  // column segments where x is more than twice an XCD's L2 (4 MB), unless the
   // format build's count tables (16 bytes per segment and row) would pass
-  // 4 GB
-  if (static_cast<int64_t>(n) * 8 >= (int64_t{16} << 20) &&
+  // 4 GB.  Row blocks against segments (us): R-MAT with x of 2.4 MB 28.4 /
+  // 31.6, 8 MB 100.7 / 93.5, 12 MB 178 / 150, 32 MB 488 / 381.
+  const int64_t x_bytes = static_cast<int64_t>(n) * 8;
+  if (x_bytes > (int64_t{8} << 20) &&
       static_cast<int64_t>(segments_for(n)) * m <= (int64_t{1} << 28)) {
     st = setup_segments(segments_for(n));
     if (st == SBLAS_ERR_ALLOC || st == SBLAS_ERR_UNSUPPORTED) {
@@ -1044,10 +1056,29 @@ int Plan::choose_csr(const std::vector<int> &h_rp) {
   std::vector<float> ms;
   if ((st = trial(forms, ms)) != SBLAS_OK) return st;
   tuned = 2;
+  for (size_t f = 0; f < forms.size(); f++) trial_ms[f] = ms[f];
+  // Narrow values: the forms over row blocks may gather x from an FP32 copy
+  // (normwise error 2.2e-8), the CSR5-style and column-sorted forms read x in
+  // FP64.  The copy is taken only where it clearly pays, so a matrix whose
+  // forms tie does not get one accuracy or the other by the noise of a trial:
+  // row blocks or segments a tenth ahead of the column-sorted form on x of
+  // 16 MB or more (R-MAT scale 22 0.6 of it, four a row in a band 0.83), row
+  // blocks 15 % ahead on smaller x with rows that are not very uneven (power
+  // law, 200,000 rows 0.75; banded, 100,000 rows of 140 0.87: FP64).  R-MAT
+  // matrices of smaller x (row CV about 9) keep FP64: the copy is worth 1 to
+  // 8 % there.
+  const bool auto_x = val_type != SBLAS_VAL_F64 && narrow == 0;
+  if (auto_x) {
+    if (x_bytes >= (int64_t{16} << 20))
+      rows_x32 = std::min(ms[0], forms.size() > 3 ? ms[3] : ms[0]) < 0.9f * ms[2];
+    else
+      rows_x32 = stats.cv < 6.0 && ms[0] < 0.85f * ms[2];
+  }
+  const bool only_rows = auto_x && rows_x32;
   size_t best = 0;
-  for (size_t f = 0; f < forms.size(); f++) {
-    trial_ms[f] = ms[f];
-    if (ms[f] < ms[best]) best = f;
+  for (size_t f = 1; f < forms.size(); f++) {
+    const bool rows = f == 3;
+    if (ms[f] < ms[best] && (rows || !only_rows)) best = f;
   }
   kernel = forms[best].first;
   variant = forms[best].second;
@@ -1055,7 +1086,7 @@ int Plan::choose_csr(const std::vector<int> &h_rp) {
   if (variant != 4) drop_sorted();
   if (variant != 6 && !seg.buffers.empty()) drop_segments();
   std::lock_guard<std::mutex> lk(g_tune_mu);
-  g_tune_cache[key] = TuneResult{kernel, variant, {trial_ms[0], trial_ms[1], trial_ms[2], trial_ms[3]}};
+  g_tune_cache[key] = TuneResult{kernel, variant, rows_x32, {trial_ms[0], trial_ms[1], trial_ms[2], trial_ms[3]}};
   return SBLAS_OK;
 }
 

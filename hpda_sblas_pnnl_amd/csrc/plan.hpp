@@ -117,6 +117,7 @@ struct Plan {
   float trial_ms[4] = {0.f, 0.f, 0.f, 0.f};
   // FP32 copy of x for row blocks over narrow values (narrow_x = 2); nullptr: FP64 x
   float *x32_rows = nullptr;
+  bool rows_x32 = true;  // auto setting of narrow_x for row blocks (a trial may clear it)
   int launches = 0;
 
   // kernel timing (measurement only)
@@ -138,6 +139,7 @@ struct Plan {
   bool has_merge(int k) const;
   int setup_tiles();
   int setup_csr5(const std::vector<int> &h_rp);
+  int narrow_x_asked() const;
   int finish_csr(const std::vector<int> &h_rp);
   int choose_csr(const std::vector<int> &h_rp);
   void free_buffers_from(size_t first);

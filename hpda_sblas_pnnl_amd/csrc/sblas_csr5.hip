@@ -25,6 +25,7 @@
 //     and no floating-point atomics are used (it adds tile carries with
 //     atomicAdd, :350,377), so results do not depend on scheduling.
 #include "internal.hpp"
+#include "span_device.hpp"
 
 namespace sblas {
 namespace {
@@ -42,59 +43,6 @@ __device__ __forceinline__ double c5_val(const uint16_t *p, int64_t j) {
 
 __device__ __forceinline__ double c5_axpby(double alpha, double s, double beta, double yv) {
   return (beta == 0.0) ? alpha * s : alpha * s + beta * yv;
-}
-
-// Wave-wide scans on DPP lane moves.  Lanes whose source lies outside the
-// move (row_shr past a 16-lane row start, rows that a broadcast does not
-// reach) read 0, the identity of both scans.
-//   row_shr:d   lane l reads l-d inside its row of 16 (d = 1, 2, 4, 8)
-//   row_bcast15 rows 1 and 3 read lane 15 of the row before (row mask 0xa)
-//   row_bcast31 rows 2 and 3 read lane 31 (row mask 0xc)
-// so after the four in-row steps each lane holds its row prefix, and the two
-// broadcasts add the totals of the rows before it.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double dpp_mov(double v) {
-  return __builtin_amdgcn_update_dpp(0.0, v, CTRL, ROWS, 0xf, false);
-}
-template <int CTRL, int ROWS>
-__device__ __forceinline__ int dpp_mov(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
-}
-constexpr int kRowShr1 = 0x111, kRowShr2 = 0x112, kRowShr4 = 0x114, kRowShr8 = 0x118;
-constexpr int kRowBcast15 = 0x142, kRowBcast31 = 0x143;
-
-// inclusive prefix sum over the 64 lanes
-__device__ __forceinline__ int wave_incl_sum(int v) {
-  v += dpp_mov<kRowShr1, 0xf>(v);
-  v += dpp_mov<kRowShr2, 0xf>(v);
-  v += dpp_mov<kRowShr4, 0xf>(v);
-  v += dpp_mov<kRowShr8, 0xf>(v);
-  v += dpp_mov<kRowBcast15, 0xa>(v);
-  v += dpp_mov<kRowBcast31, 0xc>(v);
-  return v;
-}
-
-// One step of the segmented scan: (v, head) absorbs the moved-in partner
-// unless a segment already begins inside this lane's range.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ void seg_step(double &v, int &head) {
-  const double vu = dpp_mov<CTRL, ROWS>(v);
-  const int hu = dpp_mov<CTRL, ROWS>(head);
-  if (!head) {
-    v += vu;
-    head = hu;
-  }
-}
-
-// inclusive segmented sum over the 64 lanes; head = 1 opens a segment
-__device__ __forceinline__ double wave_seg_sum(double v, int head) {
-  seg_step<kRowShr1, 0xf>(v, head);
-  seg_step<kRowShr2, 0xf>(v, head);
-  seg_step<kRowShr4, 0xf>(v, head);
-  seg_step<kRowShr8, 0xf>(v, head);
-  seg_step<kRowBcast15, 0xa>(v, head);
-  seg_step<kRowBcast31, 0xc>(v, head);
-  return v;
 }
 
 // One tile by one wave: rows closed inside the tile are written; the tile's
@@ -129,7 +77,7 @@ __device__ __forceinline__ void csr5_tile(
 
   // rank of this lane's first row start among the tile's row starts
   const int cnt = __popc(f);
-  const int incl = wave_incl_sum(cnt);
+  const int incl = span::wave_incl_sum(cnt);
   const int excl = incl - cnt;
   const int total_starts = __builtin_amdgcn_readlane(incl, 63);
 
@@ -159,8 +107,8 @@ __device__ __forceinline__ void csr5_tile(
   // segmented inclusive scan of a; a segment begins after each lane with a
   // start (lane 0 always begins one)
   const unsigned long long starts_mask = __ballot(has_start);
-  const int head = (lane == 0) ? 1 : static_cast<int>((starts_mask >> (lane - 1)) & 1ull);
-  const double sv = wave_seg_sum(a, head);
+  int head = (lane == 0) ? 1 : static_cast<int>((starts_mask >> (lane - 1)) & 1ull);
+  const double sv = span::wave_seg_sum(a, head);
   const unsigned long long below = starts_mask & ((1ull << lane) - 1ull);
   const int prev = below ? 63 - __clzll(static_cast<long long>(below)) : -1;
   const double prev_last = __shfl(last, prev < 0 ? 0 : prev, 64);

@@ -15,10 +15,9 @@
 // Matrix values and column indices are streamed with non-temporal loads so
 // they do not evict x from L2 / MALL.  Products and sums are FP64 for every
 // stored value type.
-#include <type_traits>
-
 #include "internal.hpp"
 #include "rows_device.hpp"
+#include "span_device.hpp"
 
 namespace sblas {
 namespace {
@@ -142,118 +141,93 @@ __global__ __launch_bounds__(BLOCK) void k_csr_vector_mrhs(
   }
 }
 
-// LDS-staged row blocks.  Phase 1 issues every global load the block needs
-// that does not depend on another: ITEMS values and columns per thread
-// (consecutive threads on consecutive elements, so each load instruction of a
-// wave covers whole cache lines), the block's row pointers and, with
-// beta != 0, its y entries; then the x gathers.  Row pointers go to LDS and y
-// stays in registers, so the row sums (phase 2, SUBW lanes per row, products
-// read from LDS) and the y writes (phase 3, consecutive threads on consecutive
-// rows) wait on no further memory round trip.  A block that holds a piece of
-// one long row sums in registers and reduces across the whole workgroup
-// instead.  XT float: x gathered from its FP32 copy (narrow values: half the
-// bytes per gather and per cached line of x; an FP32 value times an FP32 x is
-// exact in FP64, so x's rounding is the only one added).
-template <typename VT, int ITEMS, int SUBW, int BLOCK, typename XT = double>
-__global__ __launch_bounds__(BLOCK) void k_csr_stream(
+// Row blocks.  Phase 1 issues every global load the block needs that does not
+// depend on another: ITEMS values and columns per thread (consecutive threads
+// on consecutive elements, so each load instruction of a wave covers whole
+// cache lines), the bounds of the thread's rows and, with beta != 0, their y;
+// then the x gathers, whose products go to LDS.  Phase 2 sums the rows by
+// spans of elements (span_device.hpp).  Phase 3 writes y, consecutive threads
+// on consecutive rows, from bounds that are still in registers.  XT float: x
+// gathered from its FP32 copy (narrow values: half the bytes per gather and per
+// cached line of x; an FP32 value times an FP32 x is exact in FP64, so x's
+// rounding is the only one added).
+//
+// What bounds it: the x gathers, one L2 request an element (about 2.1e11 a
+// second on this GPU), and on small matrices the chain of dependent loads.
+// Against the form that gave each row a group of lanes, with the sums in an
+// LDS array of their own (28 KB of LDS, 5 workgroups a CU; now 18.7 KB and 8),
+// us before -> now, FP64: power law 20,000 rows 8.0 -> 6.9, 200,000 rows 25.5
+// -> 22.3; R-MAT 30,000 rows 14.2 -> 10.1, 300,000 rows 38.6 -> 31.5, scale 22
+// over column segments 463 -> 442; banded 100,000 rows of 140 56.6 -> 42.7.
+template <typename VT, int ITEMS, bool BETA, typename XT>
+__global__ __launch_bounds__(span::kBlock) void k_csr_stream(
     const RowBlock *__restrict__ blocks, int nblocks, int xcd_remap,
     const int *__restrict__ rp, const int *__restrict__ col, const VT *__restrict__ val,
     const XT *__restrict__ x, double *__restrict__ y, double alpha, double beta,
     double *__restrict__ partials) {
-  constexpr int CAP = BLOCK * ITEMS;
-  constexpr int RPT = (kStreamRowsMax + BLOCK) / BLOCK;  // row pointers per thread
-  constexpr int YPT = kStreamRowsMax / BLOCK;            // rows per thread in phase 3
-  __shared__ double prod[CAP];
-  __shared__ double ysh[kStreamRowsMax];
-  __shared__ int rps[kStreamRowsMax + 1];
-  __shared__ double wsum[BLOCK / 64];
+  constexpr int B = span::kBlock;
+  constexpr int RPT = kStreamRowsMax / B;  // rows per thread
+  __shared__ span::Shared<ITEMS> sh;
   const int b = logical_block(nblocks, xcd_remap);
   if (b < 0) return;
   const RowBlock rb = blocks[b];
   const int lo = rb.lo, hi = rb.hi;
   const int t = threadIdx.x;
   const int r0 = rb.row_begin, nrows = rb.row_end - rb.row_begin;
+  span::clear_ends(sh);
 
-  // phase 1: all independent loads first.  Lanes past the window re-read its
-  // last element (same cache line) and their product is dropped by a select;
-  // row pointer and y addresses are clamped into the block's rows, so no load
-  // sits under a branch.
-  double p[ITEMS];
-  // the first row's bounds, the same for every thread (the long-row test
-  // below must be uniform over the workgroup)
-  const int rp_first = rp[r0], rp_second = rp[r0 + 1];
-  int rpv[RPT];
-#pragma unroll
-  for (int k = 0; k < RPT; k++) rpv[k] = rp[r0 + min(t + k * BLOCK, nrows)];
-  double yv[YPT];
-  if (beta != 0.0) {
-#pragma unroll
-    for (int k = 0; k < YPT; k++) yv[k] = y[r0 + min(t + k * BLOCK, nrows - 1)];
-  } else {
-#pragma unroll
-    for (int k = 0; k < YPT; k++) yv[k] = 0.0;
-  }
+  // phase 1.  Threads past the window re-read its last element (same cache
+  // line), so no load sits under a divergent branch.
+  double v[ITEMS];
+  int c[ITEMS];
   if (hi > lo) {
-    double v[ITEMS];
-    int c[ITEMS];
 #pragma unroll
     for (int k = 0; k < ITEMS; k++) {
-      const int e = min(lo + t + k * BLOCK, hi - 1);
+      const int e = min(lo + t + k * B, hi - 1);
       v[k] = load_val(val, e);
       c[k] = load_col(col, e);
     }
+  }
+  int rs[RPT], re[RPT];
+  double yv[BETA ? RPT : 1];
+#pragma unroll
+  for (int k = 0; k < RPT; k++) {
+    if (k == 0 || k * B < nrows) {
+      const int r = r0 + min(t + k * B, nrows - 1);
+      rs[k] = rp[r];
+      re[k] = rp[r + 1];
+      if constexpr (BETA) yv[k] = y[r];
+    }
+  }
+  __syncthreads();
+  if (hi > lo) {
     XT xv[ITEMS];
 #pragma unroll
     for (int k = 0; k < ITEMS; k++) xv[k] = x[c[k]];
 #pragma unroll
+    for (int k = 0; k < RPT; k++)
+      if (t + k * B < nrows && min(re[k], hi) > max(rs[k], lo))
+        span::mark_end(sh, min(re[k], hi) - 1 - lo);
+#pragma unroll
     for (int k = 0; k < ITEMS; k++)
-      p[k] = (lo + t + k * BLOCK < hi) ? v[k] * static_cast<double>(xv[k]) : 0.0;
-  } else {
-#pragma unroll
-    for (int k = 0; k < ITEMS; k++) p[k] = 0.0;
+      sh.prod[span::pos<ITEMS>(t + k * B)] = v[k] * static_cast<double>(xv[k]);
   }
-
-  if (nrows == 1 && (rp_first < lo || rp_second > hi)) {
-    // piece of a long row: register sum, wave reduction, then across waves
-    double s = 0.0;
-#pragma unroll
-    for (int k = 0; k < ITEMS; k++) s += p[k];
-    s = subwave_sum<64>(s);
-    if ((t & 63) == 0) wsum[t >> 6] = s;
-    __syncthreads();
-    if (t == 0) {
-      double tot = 0.0;
-#pragma unroll
-      for (int w = 0; w < BLOCK / 64; w++) tot += wsum[w];
-      partials[2 * b] = tot;
-    }
-    return;
-  }
-#pragma unroll
-  for (int k = 0; k < ITEMS; k++) {
-    const int e = t + k * BLOCK;
-    if (e < hi - lo) prod[e] = p[k];
-  }
-#pragma unroll
-  for (int k = 0; k < RPT; k++)
-    if (t + k * BLOCK <= nrows) rps[t + k * BLOCK] = rpv[k];
   __syncthreads();
 
-  // phase 2: one sub-wave of SUBW lanes per row, whole waves for long rows
-  rows::block_row_sums<SUBW, BLOCK>(prod, rps, nrows, lo, hi, ysh);
-  __syncthreads();
+  // phase 2
+  span::row_sums(sh);
 
   // phase 3: y for whole rows, partials for rows cut by the window
 #pragma unroll
-  for (int k = 0; k < YPT; k++) {
-    const int i = t + k * BLOCK;
+  for (int k = 0; k < RPT; k++) {
+    const int i = t + k * B;
     if (i < nrows) {
-      const double s = ysh[i];
-      const bool edge = (i == 0 || i == nrows - 1);
-      if (edge && (rps[i] < lo || rps[i + 1] > hi)) {
+      const int e = min(re[k], hi);
+      const double s = e > max(rs[k], lo) ? sh.prod[span::pos<ITEMS>(e - 1 - lo)] : 0.0;
+      if ((i == 0 || i == nrows - 1) && (rs[k] < lo || re[k] > hi)) {
         partials[2 * b + (i == 0 ? 0 : 1)] = s;
       } else {
-        y[r0 + i] = (beta == 0.0) ? alpha * s : alpha * s + beta * yv[k];
+        y[r0 + i] = BETA ? alpha * s + beta * yv[BETA ? k : 0] : alpha * s;
       }
     }
   }
@@ -366,55 +340,30 @@ int launch_mrhs_typed(int k, const VectorLaunch &L, const DevChunk *chunks, int 
   }
 }
 
-template <typename VT, int ITEMS>
+template <typename VT, int ITEMS, typename XT>
 int launch_stream_items(const StreamLaunch &L, const RowBlock *blocks, const int *rp,
-                        const int *col, const VT *val, const double *x, double *y,
-                        double alpha, double beta, double *partials, hipStream_t s,
-                        const float *x32) {
-  constexpr int B = kStreamBlock;
-  const dim3 grid(L.grid), block(B);
-#define SBLAS_STREAM_CASE(W)                                                              \
-  case W:                                                                                 \
-    if constexpr (!std::is_same<VT, double>::value) {                                     \
-      if (x32) {                                                                          \
-        hipLaunchKernelGGL((k_csr_stream<VT, ITEMS, W, B, float>), grid, block, 0, s,     \
-                           blocks, L.nblocks, L.xcd_remap, rp, col, val, x32, y, alpha,   \
-                           beta, partials);                                               \
-        break;                                                                            \
-      }                                                                                   \
-    }                                                                                     \
-    hipLaunchKernelGGL((k_csr_stream<VT, ITEMS, W, B>), grid, block, 0, s, blocks,        \
-                       L.nblocks, L.xcd_remap, rp, col, val, x, y, alpha, beta, partials); \
-    break;
-  switch (L.subwave) {
-    SBLAS_STREAM_CASE(1)
-    SBLAS_STREAM_CASE(2)
-    SBLAS_STREAM_CASE(4)
-    SBLAS_STREAM_CASE(8)
-    SBLAS_STREAM_CASE(16)
-    SBLAS_STREAM_CASE(32)
-    SBLAS_STREAM_CASE(64)
-    default:
-      set_error(SBLAS_ERR_ARGS, "stream kernel: sub-wave must be a power of two in [1,64]");
-      return SBLAS_ERR_ARGS;
-  }
-#undef SBLAS_STREAM_CASE
+                        const int *col, const VT *val, const XT *x, double *y, double alpha,
+                        double beta, double *partials, hipStream_t s) {
+  const dim3 grid(L.grid), block(span::kBlock);
+  if (beta != 0.0)
+    hipLaunchKernelGGL((k_csr_stream<VT, ITEMS, true, XT>), grid, block, 0, s, blocks, L.nblocks,
+                       L.xcd_remap, rp, col, val, x, y, alpha, beta, partials);
+  else
+    hipLaunchKernelGGL((k_csr_stream<VT, ITEMS, false, XT>), grid, block, 0, s, blocks, L.nblocks,
+                       L.xcd_remap, rp, col, val, x, y, alpha, beta, partials);
   SBLAS_HIP_TRY(hipGetLastError());
   return SBLAS_OK;
 }
 
-template <typename VT>
+template <typename VT, typename XT>
 int launch_stream_typed(const StreamLaunch &L, const RowBlock *blocks, const int *rp,
-                        const int *col, const VT *val, const double *x, double *y,
-                        double alpha, double beta, double *partials, hipStream_t s,
-                        const float *x32) {
+                        const int *col, const VT *val, const XT *x, double *y, double alpha,
+                        double beta, double *partials, hipStream_t s) {
   switch (L.items) {
     case 8:
-      return launch_stream_items<VT, 8>(L, blocks, rp, col, val, x, y, alpha, beta, partials, s,
-                                        x32);
+      return launch_stream_items<VT, 8>(L, blocks, rp, col, val, x, y, alpha, beta, partials, s);
     case 16:
-      return launch_stream_items<VT, 16>(L, blocks, rp, col, val, x, y, alpha, beta, partials,
-                                         s, x32);
+      return launch_stream_items<VT, 16>(L, blocks, rp, col, val, x, y, alpha, beta, partials, s);
     default:
       set_error(SBLAS_ERR_ARGS, "stream kernel: items per thread must be 8 or 16");
       return SBLAS_ERR_ARGS;
@@ -428,16 +377,18 @@ int launch_csr_stream(int val_type, const StreamLaunch &L, const RowBlock *block
                       double *y, double alpha, double beta, double *partials, hipStream_t s,
                       const float *x32) {
   if (L.grid <= 0) return SBLAS_OK;
+  const float *v32 = static_cast<const float *>(val);
+  const uint16_t *v16 = static_cast<const uint16_t *>(val);
   switch (val_type) {
     case SBLAS_VAL_F64:
       return launch_stream_typed(L, blocks, rp, col, static_cast<const double *>(val), x, y,
-                                 alpha, beta, partials, s, nullptr);
+                                 alpha, beta, partials, s);
     case SBLAS_VAL_F32:
-      return launch_stream_typed(L, blocks, rp, col, static_cast<const float *>(val), x, y,
-                                 alpha, beta, partials, s, x32);
+      return x32 ? launch_stream_typed(L, blocks, rp, col, v32, x32, y, alpha, beta, partials, s)
+                 : launch_stream_typed(L, blocks, rp, col, v32, x, y, alpha, beta, partials, s);
     case SBLAS_VAL_BF16:
-      return launch_stream_typed(L, blocks, rp, col, static_cast<const uint16_t *>(val), x, y,
-                                 alpha, beta, partials, s, x32);
+      return x32 ? launch_stream_typed(L, blocks, rp, col, v16, x32, y, alpha, beta, partials, s)
+                 : launch_stream_typed(L, blocks, rp, col, v16, x, y, alpha, beta, partials, s);
     default:
       set_error(SBLAS_ERR_ARGS, "unknown value type");
       return SBLAS_ERR_ARGS;
