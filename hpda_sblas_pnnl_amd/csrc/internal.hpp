@@ -47,7 +47,8 @@ struct TileCarry {
   int head_row;   // -1: first segment began in this block
   int tail_row;   // -1: last segment ends in this block
   int spanning;   // 1: the whole block lies inside one row (head only)
-  int pad_;
+  int row0;       // merge path: the tile's first row, written before the
+                  // products (launch_merge_rows) and left alone by them
 };
 
 // Row block of the LDS-staged CSR kernel: rows [row_begin, row_end) and the
@@ -192,11 +193,13 @@ constexpr int kTileBlock = 256;   // threads per tile block
 constexpr int kTileItems = 8;     // merge items (or COO elements) per thread per tile
 constexpr int kTileSize = kTileBlock * kTileItems;
 
-int tile_subwave(double mean_row);  // 1, 4, 16 or 64 lanes per row
-int launch_csr_merge_path(int val_type, int sub, int m, int64_t nnz, int tiles, const int *rp,
+// carry[b].row0 of every merge-path tile (before the first product over carry)
+int launch_merge_rows(int m, int64_t nnz, int tiles, const int *rp, TileCarry *carry,
+                      hipStream_t s);
+int launch_csr_merge_path(int val_type, int m, int64_t nnz, int tiles, const int *rp,
                           const int *col, const void *val, const double *x, double *y,
                           double alpha, double beta, TileCarry *carry, hipStream_t s);
-int launch_coo_tiles(int val_type, int sub, int m, int64_t nnz, int tiles, const int *row_idx,
+int launch_coo_tiles(int val_type, int m, int64_t nnz, int tiles, const int *row_idx,
                      const int *col_idx, const void *val, const double *x, double *y,
                      double alpha, double beta, TileCarry *carry, hipStream_t s);
 int launch_tile_fixup(int tiles, const TileCarry *carry, double *y, double alpha, double beta,
@@ -341,6 +344,9 @@ int launch_csr5(int val_type, int sigma, int ntiles, int64_t nnz, const uint32_t
                 hipStream_t s);
 int launch_csr5_transpose(int val_type, int sigma, int64_t padded, int64_t nnz, const int *col,
                           const void *val, int *colT, void *valT, hipStream_t s);
-int launch_scale_rows(int count, const int *rows, double beta, double *y, hipStream_t s);
+// Rows cut by workgroup edges (carries 0: left to the caller) and rows without
+// elements, after launch_csr5.
+int launch_csr5_finish(int carries, const TileCarry *carry, int empty, const int *empty_rows,
+                       double alpha, double beta, double *y, hipStream_t s);
 
 }  // namespace sblas

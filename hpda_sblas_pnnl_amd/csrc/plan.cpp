@@ -422,21 +422,22 @@ int Plan::run_spmm(int k, double alpha, const double *X, double beta, double *Y,
     if (tiles == 0)
       st = launch_scale(m, beta, Y, s);
     else if (kernel == SBLAS_KERNEL_CSR5) {
-      st = launch_scale_rows(c5_empty, d_c5_empty, beta, Y, s);
+      st = launch_csr5(val_type, sigma, tiles, nnz, d_c5_tile_nz, d_c5_flags, d_c5_rows_nz,
+                       d_c5_colT, d_c5_valT, X, Y, alpha, beta, d_carry, s);
       if (st == SBLAS_OK)
-        st = launch_csr5(val_type, sigma, tiles, nnz, d_c5_tile_nz, d_c5_flags, d_c5_rows_nz,
-                         d_c5_colT, d_c5_valT, X, Y, alpha, beta, d_carry, s);
+        st = launch_csr5_finish(merge_enabled ? carry_count() : 0, d_carry, c5_empty, d_c5_empty,
+                                alpha, beta, Y, s);
     } else if (kernel == SBLAS_KERNEL_COO)
-      st = launch_coo_tiles(val_type, tile_sub, m, nnz, tiles, a0, a1, val, X, Y, alpha, beta,
-                            d_carry, s);
+      st = launch_coo_tiles(val_type, m, nnz, tiles, a0, a1, val, X, Y, alpha, beta, d_carry, s);
     else
-      st = launch_csr_merge_path(val_type, tile_sub, m, nnz, tiles, a0, a1, val, X, Y, alpha,
-                                 beta, d_carry, s);
+      st = launch_csr_merge_path(val_type, m, nnz, tiles, a0, a1, val, X, Y, alpha, beta, d_carry,
+                                 s);
     if (st != SBLAS_OK) return st;
     if (te) SBLAS_HIP_TRY(hipEventRecord(te[1], s));
     launches++;
     if (tiles > 0 && merge_enabled) {
-      st = launch_tile_fixup(carry_count(), d_carry, Y, alpha, beta, s);
+      if (kernel != SBLAS_KERNEL_CSR5)
+        st = launch_tile_fixup(carry_count(), d_carry, Y, alpha, beta, s);
       launches++;
     }
     return st;
@@ -564,12 +565,15 @@ int Plan::run_spmm(int k, double alpha, const double *X, double beta, double *Y,
 int Plan::setup_tiles() {
   const int64_t items = (kernel == SBLAS_KERNEL_COO) ? nnz : static_cast<int64_t>(m) + nnz;
   tiles = static_cast<int>((items + kTileSize - 1) / kTileSize);
-  tile_sub = opts.subwave > 0 ? opts.subwave : tile_subwave(stats.mean);
-  if (tile_sub != 1 && tile_sub != 4 && tile_sub != 16 && tile_sub != 64) tile_sub = 16;
   d_carry = static_cast<TileCarry *>(dev_alloc(sizeof(TileCarry) * std::max(tiles, 1)));
   if (!d_carry) {
     set_error(SBLAS_ERR_ALLOC, "plan: tile carry allocation failed");
     return SBLAS_ERR_ALLOC;
+  }
+  if (kernel == SBLAS_KERNEL_MERGE) {  // the tiles' rows once, for every product
+    int st = launch_merge_rows(m, nnz, tiles, a0, d_carry, nullptr);
+    if (st != SBLAS_OK) return st;
+    SBLAS_HIP_TRY(hipStreamSynchronize(nullptr));
   }
   return SBLAS_OK;
 }

@@ -71,8 +71,6 @@ struct Plan {
   int tiles = 0;
   int sigma = 0;
   TileCarry *d_carry = nullptr;
-  int *d_tile_row = nullptr;
-  uint32_t *d_tile_flags = nullptr;
 
   // column-panel form of kernel 1 (variant 3); rows cut by chunk edges
   PanelFormat panel;
@@ -131,7 +129,6 @@ struct Plan {
   int setup_vector(const int *h_rp);
   int setup_stream(const int *h_rp);
   bool merge_enabled = true;          // false: caller launches run_merge itself
-  int tile_sub = 16;                  // lanes per row in the tile kernels
   bool uses_tiles(int k) const;
   // carries left for the ordered fix-up: one per tile, or one per workgroup
   // of four tiles for the CSR5-style kernel (its carries meet in LDS first)

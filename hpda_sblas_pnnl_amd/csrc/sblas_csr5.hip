@@ -14,8 +14,9 @@
 //     the tile comes from a prefix sum of flag counts over lanes, and the
 //     list of non-empty rows maps it to the row (empty rows are written by
 //     a separate pass);
-//   * each lane sums its segments sequentially in FP64; rows that end inside
-//     one lane are written directly;
+//   * each lane sums its segments sequentially in FP64; the sums of rows that
+//     end in the tile go to LDS by their rank and are written to y together,
+//     consecutive lanes on consecutive non-empty rows;
 //   * rows crossing lanes are finished by a segmented inclusive scan across
 //     the wave on DPP lane moves (row_shr inside 16-lane rows, row_bcast
 //     across them); the four tiles of a workgroup stage their carries in LDS
@@ -25,6 +26,7 @@
 //     and no floating-point atomics are used (it adds tile carries with
 //     atomicAdd, :350,377), so results do not depend on scheduling.
 #include "internal.hpp"
+#include "rows_device.hpp"
 #include "span_device.hpp"
 
 namespace sblas {
@@ -45,14 +47,24 @@ __device__ __forceinline__ double c5_axpby(double alpha, double s, double beta, 
   return (beta == 0.0) ? alpha * s : alpha * s + beta * yv;
 }
 
-// One tile by one wave: rows closed inside the tile are written; the tile's
-// head / tail / spanning partials go to *out (lane 0).
-template <typename VT, int SIGMA>
-__device__ __forceinline__ void csr5_tile(
+// Sums of rows closed in a tile that wait in LDS for the writes; a tile with
+// more rows than this (rows of one or two elements) writes the others from
+// their lanes.
+constexpr int kC5Rows = 512;
+
+// What one wave leaves for its writes: row sums by rank, ranks [from, count).
+struct C5Rows {
+  int first_nz, from, count;
+};
+
+// One tile by one wave: sums of rows closed inside the tile to rsum[rank]; the
+// tile's head / tail / spanning partials to *out (lane 0).
+template <typename VT, int SIGMA, bool BETA>
+__device__ __forceinline__ C5Rows csr5_tile(
     int p, int ntiles, int64_t nnz, const uint32_t *__restrict__ tile_nz,
     const uint32_t *__restrict__ flags, const int *__restrict__ rows_nz,
     const int *__restrict__ colT, const VT *__restrict__ valT, const double *__restrict__ x,
-    double *__restrict__ y, double alpha, double beta, TileCarry *out) {
+    double *__restrict__ y, double alpha, double beta, double *rsum, TileCarry *out) {
   constexpr int T = 64 * SIGMA;
   const int lane = threadIdx.x & 63;
   const int64_t base = static_cast<int64_t>(p) * T;
@@ -75,11 +87,20 @@ __device__ __forceinline__ void csr5_tile(
 #pragma unroll
   for (int s = 0; s < SIGMA; s++) xv[s] = x[c[s]];
 
-  // rank of this lane's first row start among the tile's row starts
+  // rank of this lane's first row start among the tile's row starts: start j
+  // closes the tile's row j
   const int cnt = __popc(f);
   const int incl = span::wave_incl_sum(cnt);
   const int excl = incl - cnt;
   const int total_starts = __builtin_amdgcn_readlane(incl, 63);
+  auto close = [&](int j, double s) {
+    if (j < kC5Rows) {
+      rsum[j] = s;
+    } else {
+      const int r = rows_nz[first_nz + j];
+      y[r] = c5_axpby(alpha, s, beta, BETA ? y[r] : 0.0);
+    }
+  };
 
   // in-lane segments
   const int64_t lane_first = base + static_cast<int64_t>(lane) * SIGMA;
@@ -89,12 +110,7 @@ __device__ __forceinline__ void csr5_tile(
   for (int s = 0; s < SIGMA; s++) {
     const double prod = (lane_first + s < nnz) ? v[s] * xv[s] : 0.0;
     if ((f >> s) & 1u) {
-      if (k == 0) {
-        first = cur;
-      } else {
-        const int r = rows_nz[first_nz + excl + k];
-        y[r] = c5_axpby(alpha, cur, beta, y[r]);
-      }
+      if (k == 0) first = cur; else close(excl + k, cur);
       k++;
       cur = 0.0;
     }
@@ -118,12 +134,11 @@ __device__ __forceinline__ void csr5_tile(
   int head_row = -1;
   if (has_start) {
     const double total = sv + (prev >= 0 ? prev_last : 0.0);
-    const int r = rows_nz[first_nz + excl];
     if (excl == 0 && !starts_row) {
       head_part = total;  // began in an earlier tile
-      head_row = r;
+      head_row = rows_nz[first_nz];
     } else {
-      y[r] = c5_axpby(alpha, total, beta, y[r]);
+      close(excl, total);
     }
   }
   // the segment open at the tile's end
@@ -135,29 +150,20 @@ __device__ __forceinline__ void csr5_tile(
   const int first_lane = any ? __ffsll(static_cast<long long>(any)) - 1 : 0;
   const double head_part0 = __shfl(head_part, first_lane, 64);
   const int head_row0 = __shfl(head_row, first_lane, 64);
+  const double open_sum = last_lane < 0 ? tail_scan  // no start in the tile: one segment
+                                        : open_last + (last_lane < 63 ? tail_scan : 0.0);
+  const bool open_began_before = (last_lane < 0) && !starts_row;
+  const bool closes_open = ends_row && !open_began_before;  // the open row ends with the tile
   if (lane == 0) {
+    if (closes_open) close(total_starts, open_sum);
     TileCarry cy{head_part0, 0.0, head_row0, -1, 0, 0};
     if (head_row0 < 0) cy.head = 0.0;
-    const int open_row = rows_nz[first_nz + total_starts];
-    double open_sum;
-    if (last_lane < 0) {
-      open_sum = tail_scan;  // no start in the tile: one segment from lane 0
-    } else {
-      open_sum = open_last + (last_lane < 63 ? tail_scan : 0.0);
-    }
-    const bool open_began_before = (last_lane < 0) && !starts_row;
-    if (ends_row) {
+    if (!closes_open) {
+      const int open_row = rows_nz[first_nz + total_starts];
       if (open_began_before) {
         cy.head = open_sum;
         cy.head_row = open_row;
-      } else {
-        y[open_row] = c5_axpby(alpha, open_sum, beta, y[open_row]);
-      }
-    } else {
-      if (open_began_before) {
-        cy.head = open_sum;
-        cy.head_row = open_row;
-        cy.spanning = 1;
+        cy.spanning = ends_row ? 0 : 1;
       } else {
         cy.tail = open_sum;
         cy.tail_row = open_row;
@@ -165,27 +171,42 @@ __device__ __forceinline__ void csr5_tile(
     }
     *out = cy;
   }
+  // rank 0 is the head unless the tile begins a row
+  return C5Rows{first_nz, starts_row ? 0 : 1,
+                min(total_starts + (closes_open ? 1 : 0), kC5Rows)};
 }
 
-// Four tiles per workgroup.  Their carries are staged in LDS and folded in
+// Four tiles per workgroup.  Row sums wait in LDS for the whole tile: a row
+// number looked up and y stored from inside the lanes' sums stalled the wave
+// at nearly every element (some lane closes a row there), and y was read for
+// beta == 0 too.  FP64, whole product, us before -> now: R-MAT scale 20 128 ->
+// 112, power law 1,000,003 rows 200 -> 172, 20,000 rows 12.6 -> 10.5.  Their carries are staged in LDS and folded in
 // tile order by one thread: rows that begin and end inside the workgroup are
 // written here, and one carry per workgroup (same meaning as a tile's) is
 // left for the ordered fix-up over workgroups.
-template <typename VT, int SIGMA>
+template <typename VT, int SIGMA, bool BETA>
 __global__ __launch_bounds__(256) void k_csr5(
     int ntiles, int64_t nnz, const uint32_t *__restrict__ tile_nz,
     const uint32_t *__restrict__ flags, const int *__restrict__ rows_nz,
     const int *__restrict__ colT, const VT *__restrict__ valT, const double *__restrict__ x,
     double *__restrict__ y, double alpha, double beta, TileCarry *__restrict__ carry) {
   __shared__ TileCarry wc[4];
+  __shared__ double rsum[4][kC5Rows];
+  const int b = rows::logical_block((ntiles + 3) / 4, 1);
+  if (b < 0) return;
   const int wave = threadIdx.x >> 6;
-  const int p = blockIdx.x * 4 + wave;
+  const int p = b * 4 + wave;
+  C5Rows mine{0, 0, 0};
   if (p < ntiles)  // uniform per wave; every wave reaches the barrier below
-    csr5_tile<VT, SIGMA>(p, ntiles, nnz, tile_nz, flags, rows_nz, colT, valT, x, y, alpha, beta,
-                         &wc[wave]);
+    mine = csr5_tile<VT, SIGMA, BETA>(p, ntiles, nnz, tile_nz, flags, rows_nz, colT, valT, x, y,
+                                      alpha, beta, rsum[wave], &wc[wave]);
   __syncthreads();
+  for (int j = mine.from + (static_cast<int>(threadIdx.x) & 63); j < mine.count; j += 64) {
+    const int r = rows_nz[mine.first_nz + j];
+    y[r] = c5_axpby(alpha, rsum[wave][j], beta, BETA ? y[r] : 0.0);
+  }
   if (threadIdx.x != 0) return;
-  const int count = min(4, ntiles - static_cast<int>(blockIdx.x) * 4);
+  const int count = min(4, ntiles - b * 4);
   TileCarry out{0.0, 0.0, -1, -1, 0, 0};
   bool all_span = true;
   int open = -1;  // row opened by a tile of this workgroup and not yet closed
@@ -204,14 +225,14 @@ __global__ __launch_bounds__(256) void k_csr5(
     all_span = false;
     if (c.head_row >= 0) {
       if (open >= 0) {
-        y[open] = c5_axpby(alpha, osum + c.head, beta, y[open]);
+        y[open] = c5_axpby(alpha, osum + c.head, beta, BETA ? y[open] : 0.0);
         open = -1;
       } else {
         out.head += c.head;
         out.head_row = c.head_row;
       }
     } else if (open >= 0) {
-      y[open] = c5_axpby(alpha, osum, beta, y[open]);
+      y[open] = c5_axpby(alpha, osum, beta, BETA ? y[open] : 0.0);
       open = -1;
     }
     if (c.tail_row >= 0) {
@@ -225,7 +246,7 @@ __global__ __launch_bounds__(256) void k_csr5(
     out.tail = osum;
     out.tail_row = open;
   }
-  carry[blockIdx.x] = out;
+  carry[b] = out;
 }
 
 // Transposed, zero-padded copy: element (lane l, s) of tile p moves to
@@ -244,11 +265,21 @@ __global__ void k_csr5_transpose(int64_t padded, int64_t nnz, int sigma, const i
   valT[o] = src < nnz ? val[src] : VT(0);
 }
 
-__global__ void k_scale_rows(int count, const int *__restrict__ rows, double beta,
-                             double *__restrict__ y) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= count) return;
-  const int r = rows[i];
+// After the tiles: the rows cut by workgroup edges (first fix_blocks
+// workgroups; none when the caller closes them itself) and the rows without
+// elements, in one launch.
+__global__ void k_csr5_finish(int fix_blocks, int carries, const TileCarry *__restrict__ carry,
+                              int empty, const int *__restrict__ empty_rows, double alpha,
+                              double beta, double *__restrict__ y) {
+  const int blk = blockIdx.x;
+  if (blk < fix_blocks) {
+    const int b = blk * blockDim.x + threadIdx.x;
+    if (b < carries) span::close_cut_row(b, carries, carry, y, alpha, beta);
+    return;
+  }
+  const int i = (blk - fix_blocks) * blockDim.x + threadIdx.x;
+  if (i >= empty) return;
+  const int r = empty_rows[i];
   y[r] = (beta == 0.0) ? 0.0 : beta * y[r];
 }
 
@@ -257,24 +288,25 @@ int csr5_launch_sigma(int sigma, int ntiles, int64_t nnz, const uint32_t *tile_n
                       const uint32_t *flags, const int *rows_nz, const int *colT,
                       const VT *valT, const double *x, double *y, double alpha, double beta,
                       TileCarry *carry, hipStream_t s) {
-  const dim3 grid((ntiles + 3) / 4), block(256);
+  const dim3 grid(((ntiles + 3) / 4 + 7) / 8 * 8), block(256);
+#define SBLAS_C5_CASE(S)                                                                     \
+  case S:                                                                                    \
+    if (beta != 0.0)                                                                         \
+      hipLaunchKernelGGL((k_csr5<VT, S, true>), grid, block, 0, s, ntiles, nnz, tile_nz,     \
+                         flags, rows_nz, colT, valT, x, y, alpha, beta, carry);              \
+    else                                                                                     \
+      hipLaunchKernelGGL((k_csr5<VT, S, false>), grid, block, 0, s, ntiles, nnz, tile_nz,    \
+                         flags, rows_nz, colT, valT, x, y, alpha, beta, carry);              \
+    break;
   switch (sigma) {
-    case 8:
-      hipLaunchKernelGGL((k_csr5<VT, 8>), grid, block, 0, s, ntiles, nnz, tile_nz, flags, rows_nz,
-                         colT, valT, x, y, alpha, beta, carry);
-      break;
-    case 16:
-      hipLaunchKernelGGL((k_csr5<VT, 16>), grid, block, 0, s, ntiles, nnz, tile_nz, flags,
-                         rows_nz, colT, valT, x, y, alpha, beta, carry);
-      break;
-    case 32:
-      hipLaunchKernelGGL((k_csr5<VT, 32>), grid, block, 0, s, ntiles, nnz, tile_nz, flags,
-                         rows_nz, colT, valT, x, y, alpha, beta, carry);
-      break;
+    SBLAS_C5_CASE(8)
+    SBLAS_C5_CASE(16)
+    SBLAS_C5_CASE(32)
     default:
       set_error(SBLAS_ERR_ARGS, "csr5: sigma must be 8, 16 or 32");
       return SBLAS_ERR_ARGS;
   }
+#undef SBLAS_C5_CASE
   SBLAS_HIP_TRY(hipGetLastError());
   return SBLAS_OK;
 }
@@ -325,10 +357,12 @@ int launch_csr5_transpose(int val_type, int sigma, int64_t padded, int64_t nnz, 
   return SBLAS_OK;
 }
 
-int launch_scale_rows(int count, const int *rows, double beta, double *y, hipStream_t s) {
-  if (count <= 0) return SBLAS_OK;
-  hipLaunchKernelGGL(k_scale_rows, dim3((count + 255) / 256), dim3(256), 0, s, count, rows, beta,
-                     y);
+int launch_csr5_finish(int carries, const TileCarry *carry, int empty, const int *empty_rows,
+                       double alpha, double beta, double *y, hipStream_t s) {
+  const int fix_blocks = (carries + 255) / 256, grid = fix_blocks + (empty + 255) / 256;
+  if (grid <= 0) return SBLAS_OK;
+  hipLaunchKernelGGL(k_csr5_finish, dim3(grid), dim3(256), 0, s, fix_blocks, carries, carry, empty,
+                     empty_rows, alpha, beta, y);
   SBLAS_HIP_TRY(hipGetLastError());
   return SBLAS_OK;
 }

@@ -147,5 +147,21 @@ __device__ __forceinline__ void row_sums(Shared<ITEMS> &sh) {
   __syncthreads();
 }
 
+// A row cut by tile edges whose last tile before the cut is b: the head
+// partials of the following tiles are added in order (through tiles that lie
+// wholly inside the row) and y is written once.
+__device__ __forceinline__ void close_cut_row(int b, int tiles,
+                                              const TileCarry *__restrict__ carry,
+                                              double *__restrict__ y, double alpha, double beta) {
+  const TileCarry c = carry[b];
+  if (c.tail_row < 0 || c.spanning) return;
+  const int r = c.tail_row;
+  double s = c.tail;
+  int n = b + 1;
+  while (n < tiles && carry[n].spanning) s += carry[n++].head;
+  if (n < tiles && carry[n].head_row == r) s += carry[n].head;
+  y[r] = (beta == 0.0) ? alpha * s : alpha * s + beta * y[r];
+}
+
 }  // namespace span
 }  // namespace sblas

@@ -1,6 +1,7 @@
 """Products that sum rows by spans of elements (csrc/span_device.hpp: one vector
-over row blocks; csrc/sblas_spmm.hip: several) against the FP64 oracle, at the
-sizes where spans, row ends and block edges meet.
+over row blocks, merge-path and COO tiles; csrc/sblas_spmm.hip: several vectors)
+and by CSR5-style tiles against the FP64 oracle, at the sizes where spans, row
+ends, tile and block edges meet.
 
 Bound: two sums of a row's L products in different orders, each off by at most
 (L + 3) roundings of 2^-53 of alpha * sum |a x| + |beta y| (the products, the
@@ -36,30 +37,37 @@ SHAPES = {
     "ragged": [int(v) for v in np.random.default_rng(3).geometric(0.06, 900)],
     "short_block": [3, 0, 4, 65],
     "empty": [0] * 40,
+    # tiles of row ends alone, empty runs of eight and nine, of a wave and more
+    "gaps": [0] * 4200 + [1] + [0] * 9 + [2] + [0] * 8 + [1] + [0] * 64 + [70] + [0] * 700 + [2],
+    # rows and elements together fill merge-path tiles exactly
+    "full_tile": [1] * 1024 + [3] * 1024,
 }
+
+
+def _values(count, dtype, rng):
+    """Values as the oracle and the device hold them."""
+    import torch
+    from hpda_sblas_pnnl_amd import gen as G
+    wide = rng.standard_normal(count)
+    if dtype == "f64":
+        return wide, torch.from_numpy(wide).cuda()
+    if dtype == "f32":
+        return (wide.astype(np.float32).astype(np.float64),
+                torch.from_numpy(wide.astype(np.float32)).cuda())
+    bits = G.to_bf16_bits(wide)
+    return G.from_bf16_bits(bits), torch.from_numpy(bits.view(np.int16)).cuda()
 
 
 @pytest.mark.parametrize("shape", list(SHAPES))
 @pytest.mark.parametrize("k", [1, 2, 4, 8, 16])
 def test_row_blocks(oracle, shape, k):
     import torch
-    from hpda_sblas_pnnl_amd import gen as G
     from hpda_sblas_pnnl_amd.device import SpmvPlan
     rng = np.random.default_rng(17 * k + len(shape))
     lens, n = SHAPES[shape], 6000
     m = len(lens)
     rp, col = _rows(lens, n, rng)
-    wide = rng.standard_normal(len(col))
-    dtype = DTYPES[(k + len(shape)) % 3]
-    if dtype == "f64":
-        val, dval = wide, torch.from_numpy(wide).cuda()
-    elif dtype == "f32":
-        val = wide.astype(np.float32).astype(np.float64)
-        dval = torch.from_numpy(wide.astype(np.float32)).cuda()
-    else:
-        bits = G.to_bf16_bits(wide)
-        val = G.from_bf16_bits(bits)
-        dval = torch.from_numpy(bits.view(np.int16)).cuda()
+    val, dval = _values(len(col), DTYPES[(k + len(shape)) % 3], rng)
     X, Y0 = rng.uniform(-1, 1, (n, k)), rng.uniform(-1, 1, (m, k))
     absx = oracle.csr_spmm(m, k, np.abs(val), rp, col, np.abs(X), 1.0, 0.0, np.zeros((m, k)))
     # X and Y start 8 bytes past a 16-byte boundary
@@ -79,3 +87,40 @@ def test_row_blocks(oracle, shape, k):
             bound = 2 * (np.asarray(lens)[:, None] + 3) * EPS * scale
             assert (np.abs(dY.cpu().numpy() - ref) <= bound).all()
             assert buf[0] == 7.0 and (buf[m * k + 1:] == 7.0).all()
+
+
+@pytest.mark.parametrize("shape", list(SHAPES))
+@pytest.mark.parametrize("form", ["merge", "coo", "csr5_8", "csr5_16", "csr5_32"])
+def test_tiles(oracle, shape, form):
+    import torch
+    from hpda_sblas_pnnl_amd.device import SpmvPlan
+    lens, n = SHAPES[shape], 6000
+    m = len(lens)
+    if form == "coo" and sum(lens) == 0:
+        pytest.skip("a COO plan takes its row indices' address")
+    rng = np.random.default_rng(5 * len(form) + len(shape))
+    rp, col = _rows(lens, n, rng)
+    val, dval = _values(len(col), DTYPES[(len(form) + len(shape)) % 3], rng)
+    x, y0 = rng.uniform(-1, 1, n), rng.uniform(-1, 1, m)
+    absx = oracle.csr_spmv(m, n, np.abs(val), rp, col, np.abs(x), 1.0, 0.0, np.zeros(m))
+    dx = torch.from_numpy(x).cuda()
+    dcol = torch.from_numpy(col).cuda()
+    if form == "coo":
+        rows = torch.from_numpy(np.repeat(np.arange(m, dtype=np.int32), lens)).cuda()
+        plan = SpmvPlan("coo", m, n, rows, dcol, dval, kernel="coo")
+    else:
+        kernel, _, sigma = form.partition("_")
+        plan = SpmvPlan("csr", m, n, torch.from_numpy(rp).cuda(), dcol, dval, kernel=kernel,
+                        sigma=int(sigma or 0))
+    for alpha, beta in ((1.0, 0.0), (-0.75, 0.5)):
+        buf = torch.full((m + 3,), 7.0, dtype=torch.float64, device="cuda")
+        dy = buf[1:m + 1]
+        dy.copy_(torch.from_numpy(y0))
+        if beta == 0.0:
+            dy.fill_(float("nan"))  # beta == 0 does not read y
+        plan.spmv(dx, dy, alpha, beta)
+        ref = oracle.csr_spmv(m, n, val, rp, col, x, alpha, beta, y0)
+        scale = abs(alpha) * absx + abs(beta) * np.abs(y0)
+        bound = 2 * (np.asarray(lens) + 3) * EPS * scale
+        assert (np.abs(dy.cpu().numpy() - ref) <= bound).all()
+        assert buf[0] == 7.0 and (buf[m + 1:] == 7.0).all()
