@@ -158,13 +158,15 @@ struct sblas_batch_s {
       if (grid_panel > 0 && ps != s) SBLAS_HIP_TRY(hipStreamWaitEvent(ps, fork, 0));
       if (grid_rows > 0 && rs != s) SBLAS_HIP_TRY(hipStreamWaitEvent(rs, fork, 0));
     }
-    // beside the matrices with launches of their own, the row blocks run one
-    // item per workgroup, so CUs pass to those launches as items finish (a
-    // persistent launch held every CU for 1.9 ms while they waited: 64-matrix
-    // FP32 batch 4.66 ms, 4.49 ms this way); SBLAS_BATCH_FLAT overrides (0
+    // row blocks run one item per workgroup: the hardware hands out
+    // workgroups as CUs free up, where the persistent launch takes 107
+    // registers (four workgroups a CU against eight) and pays a counter round
+    // trip an item (us, persistent / flat: twelve matrices of 5,000 to 60,000
+    // rows, FP64 202 / 66; eight of 40,000 to 300,000 441 / 285; sixteen of
+    // 10,000 to 1,000,000 798 / 691).  SBLAS_BATCH_FLAT overrides (0
     // persistent, 1 flat row blocks, 2 flat row panels too)
     int flat = sblas::env_int_b("SBLAS_BATCH_FLAT", -1);
-    if (flat < 0) flat = solo.empty() ? 0 : 1;
+    if (flat < 0) flat = 1;
     st = sblas::launch_batch(sblas::kBatchPanel, items_per_thread, grid_panel, n_panel,
                                  d_items, d_mats, d_partials, d_qbound, d_ctr, ps, flat >= 2);
     if (st != SBLAS_OK) return st;

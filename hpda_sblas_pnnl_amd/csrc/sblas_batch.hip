@@ -14,151 +14,34 @@
 // partials that one merge launch combines in item order.
 #include "internal.hpp"
 #include "panel_device.hpp"
+#include "row_block_device.hpp"
 
 namespace sblas {
 namespace {
-
-__device__ __forceinline__ double t_val(const double *p, int j) {
-  return __builtin_nontemporal_load(p + j);
-}
-__device__ __forceinline__ double t_val(const float *p, int j) {
-  return static_cast<double>(__builtin_nontemporal_load(p + j));
-}
-__device__ __forceinline__ double t_val(const uint16_t *p, int j) {
-  const uint32_t h = __builtin_nontemporal_load(p + j);
-  return static_cast<double>(__uint_as_float(h << 16));
-}
 
 __device__ __forceinline__ double b_axpby(double alpha, double s, double beta, double yv) {
   return (beta == 0.0) ? alpha * s : alpha * s + beta * yv;
 }
 
-// One row block (the LDS-staged form of kernel 1): products of the block's
-// element window into LDS, sub-wave row sums, y written (or the partials of
-// rows the window cuts).  lds holds BLOCK*ITEMS + kStreamRowsMax doubles.
-template <typename VT, int ITEMS, int BLOCK>
-__device__ __forceinline__ void row_block(int w, const BatchItem &it, const BatchMatrix &M,
-                                          double *__restrict__ partials, double *lds,
-                                          double *wsum) {
-  const VT *__restrict__ val = static_cast<const VT *>(M.val);
-  constexpr int CAP = BLOCK * ITEMS;
-  double *prod = lds;
-  double *ysh = lds + CAP;
-  const int t = threadIdx.x;
-  const int *__restrict__ rp = M.rp;
-  const int *__restrict__ col = M.col;
-  const double *__restrict__ x = M.x;
-  double *__restrict__ y = M.y;
-  const int lo = it.lo, hi = it.hi;
-  double p[ITEMS];
-  if (hi > lo) {
-    double v[ITEMS];
-    int c[ITEMS];
-#pragma unroll
-    for (int k = 0; k < ITEMS; k++) {
-      const int e = min(lo + t + k * BLOCK, hi - 1);
-      v[k] = t_val(val, e);
-      c[k] = __builtin_nontemporal_load(col + e);
-    }
-    double xv[ITEMS];
-    if (sizeof(VT) < 8 && M.x32) {
-      // FP32 copy: 4-byte gathers, half the lines of x; an FP32 value times
-      // an FP32 x is exact in FP64, so x's rounding is the only one added
-      float xf[ITEMS];
-#pragma unroll
-      for (int k = 0; k < ITEMS; k++) xf[k] = M.x32[c[k]];
-#pragma unroll
-      for (int k = 0; k < ITEMS; k++) xv[k] = static_cast<double>(xf[k]);
-    } else {
-#pragma unroll
-      for (int k = 0; k < ITEMS; k++) xv[k] = x[c[k]];
-    }
-#pragma unroll
-    for (int k = 0; k < ITEMS; k++) p[k] = (lo + t + k * BLOCK < hi) ? v[k] * xv[k] : 0.0;
-  } else {
-#pragma unroll
-    for (int k = 0; k < ITEMS; k++) p[k] = 0.0;
-  }
-  const int nrows = it.row_end - it.row_begin;
-  if (nrows == 1 && (rp[it.row_begin] < lo || rp[it.row_begin + 1] > hi)) {
-    double s = 0.0;
-#pragma unroll
-    for (int k = 0; k < ITEMS; k++) s += p[k];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    if ((t & 63) == 0) wsum[t >> 6] = s;
-    __syncthreads();
-    if (t == 0) {
-      double tot = 0.0;
-#pragma unroll
-      for (int q = 0; q < BLOCK / 64; q++) tot += wsum[q];
-      partials[it.pslot] = tot;
-    }
-    __syncthreads();
-    return;
-  }
-#pragma unroll
-  for (int k = 0; k < ITEMS; k++) {
-    const int e = t + k * BLOCK;
-    if (e < hi - lo) prod[e] = p[k];
-  }
-  __syncthreads();
-  // row sums: one sub-wave per row; a row of more than 16 sub-wave widths is
-  // left to whole waves afterwards (found by a ballot over the block's rows,
-  // the same list in every wave, dealt out in turn), so a long row never
-  // holds the block for len / sub steps
-  const int sub = M.subwave;  // 1..64, power of two
-  const int subs = BLOCK / sub;
-  const int g = t / sub, lane = t % sub;
-  const int longest = 16 * sub;
-  for (int i = g; i < nrows; i += subs) {
-    const int r = it.row_begin + i;
-    const int s0 = max(rp[r], lo) - lo, e0 = min(rp[r + 1], hi) - lo;
-    if (sub < 64 && e0 - s0 > longest) continue;
-    double s = 0.0;
-    for (int j = s0 + lane; j < e0; j += sub) s += prod[j];
-    for (int off = sub >> 1; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    if (lane == 0) ysh[i] = s;
-  }
-  if (sub < 64) {
-    const int w = t >> 6, l = t & 63;
-    int seen = 0;
-    for (int base = 0; base < nrows; base += 64) {
-      const int i = base + l;
-      bool is_long = false;
-      if (i < nrows) {
-        const int r = it.row_begin + i;
-        is_long = min(rp[r + 1], hi) - max(rp[r], lo) > longest;
-      }
-      uint64_t mask = __ballot(is_long);
-      while (mask) {
-        const int bit = __ffsll(static_cast<unsigned long long>(mask)) - 1;
-        mask &= mask - 1;
-        if (seen % (BLOCK / 64) == w) {
-          const int r = it.row_begin + base + bit;
-          const int s0 = max(rp[r], lo) - lo, e0 = min(rp[r + 1], hi) - lo;
-          double s = 0.0;
-          for (int j = s0 + l; j < e0; j += 64) s += prod[j];
-#pragma unroll
-          for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-          if (l == 0) ysh[base + bit] = s;
-        }
-        seen++;
-      }
+// One row block of one vector (row_block_device.hpp): x from its FP32 copy
+// where the matrix has one.
+template <typename VT, int ITEMS>
+__device__ __forceinline__ void row_block(const BatchItem &it, const BatchMatrix &M,
+                                          double *__restrict__ partials,
+                                          span::Shared<ITEMS> &sh) {
+  const RowBlock rb{it.row_begin, it.row_end, it.lo, it.hi};
+  const VT *val = static_cast<const VT *>(M.val);
+  double *slots = partials + it.pslot;
+  const bool with_beta = M.beta != 0.0;
+  if constexpr (sizeof(VT) < 8) {
+    if (M.x32) {
+      rows::row_block<VT, ITEMS, float>(rb, with_beta, M.rp, M.col, val, M.x32, M.y, M.alpha,
+                                        M.beta, slots, sh);
+      return;
     }
   }
-  __syncthreads();
-  for (int i = t; i < nrows; i += BLOCK) {
-    const int r = it.row_begin + i;
-    const double s = ysh[i];
-    const bool edge = (i == 0 || i == nrows - 1);
-    if (edge && (rp[r] < lo || rp[r + 1] > hi)) {
-      partials[it.pslot + (i == 0 ? 0 : 1)] = s;
-    } else {
-      y[r] = b_axpby(M.alpha, s, M.beta, y[r]);
-    }
-  }
-  __syncthreads();
+  rows::row_block<VT, ITEMS, double>(rb, with_beta, M.rp, M.col, val, M.x, M.y, M.alpha, M.beta,
+                                     slots, sh);
 }
 
 // One row block with K right-hand sides (X n x K, Y m x K, row-major): lane
@@ -186,8 +69,8 @@ __device__ __forceinline__ void row_block_mrhs(const BatchItem &it, const BatchM
       int c[4];
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        v[i] = t_val(val, j + i * step);
-        c[i] = __builtin_nontemporal_load(col + j + i * step);
+        v[i] = rows::load_val(val, j + i * step);
+        c[i] = rows::load_col(col, j + i * step);
       }
       double xv[4];
 #pragma unroll
@@ -196,7 +79,7 @@ __device__ __forceinline__ void row_block_mrhs(const BatchItem &it, const BatchM
       for (int i = 0; i < 4; i++) sum += v[i] * xv[i];
     }
     for (; j < j1; j += step)
-      sum += t_val(val, j) * X[static_cast<int64_t>(col[j]) * K + vec];
+      sum += rows::load_val(val, j) * X[static_cast<int64_t>(col[j]) * K + vec];
     return sum;
   };
   const int nrows = it.row_end - it.row_begin;
@@ -300,15 +183,16 @@ __device__ __forceinline__ void row_panel_any(const BatchItem &it, const BatchMa
 
 // A row-block item of one value type: one vector or K right-hand sides.
 template <typename VT, int ITEMS, int BLOCK>
-__device__ __forceinline__ void rows_typed(int w, const BatchItem &it, const BatchMatrix &M,
-                                           double *__restrict__ partials, double *lds,
-                                           double *wsum) {
+__device__ __forceinline__ void rows_typed(const BatchItem &it, const BatchMatrix &M,
+                                           double *__restrict__ partials, double *lds) {
   switch (M.k) {  // 1, 2, 4, 8 or 16 (checked when the batch is created)
     case 2: row_block_mrhs<VT, 2, BLOCK>(it, M, partials, lds); break;
     case 4: row_block_mrhs<VT, 4, BLOCK>(it, M, partials, lds); break;
     case 8: row_block_mrhs<VT, 8, BLOCK>(it, M, partials, lds); break;
     case 16: row_block_mrhs<VT, 16, BLOCK>(it, M, partials, lds); break;
-    default: row_block<VT, ITEMS, BLOCK>(w, it, M, partials, lds, wsum); break;
+    default:
+      row_block<VT, ITEMS>(it, M, partials, *reinterpret_cast<span::Shared<ITEMS> *>(lds));
+      break;
   }
 }
 
@@ -316,25 +200,24 @@ __device__ __forceinline__ void rows_typed(int w, const BatchItem &it, const Bat
 template <int MODE, int ITEMS, int BLOCK>
 __host__ __device__ constexpr int batch_lds() {
   return MODE == kBatchPanel ? panel::lds_doubles<uint16_t, kBatchPanelRowsMax / 256>()
-                             : BLOCK * ITEMS + kStreamRowsMax;
+                             : static_cast<int>(sizeof(span::Shared<ITEMS>) / sizeof(double));
 }
 
 // work item w of the list
 template <int MODE, int ITEMS, int BLOCK>
 __device__ __forceinline__ void batch_item(int w, const BatchItem *__restrict__ items,
                                            const BatchMatrix *__restrict__ mats,
-                                           double *__restrict__ partials, double *lds,
-                                           double *wsum) {
+                                           double *__restrict__ partials, double *lds) {
   const BatchItem it = items[w];
   const BatchMatrix &M = mats[it.mat];
   if constexpr (MODE == kBatchPanel) {
     row_panel_any(it, M, partials, lds);
   } else if (M.val_type == SBLAS_VAL_F64) {  // value type chosen once per item
-    rows_typed<double, ITEMS, BLOCK>(w, it, M, partials, lds, wsum);
+    rows_typed<double, ITEMS, BLOCK>(it, M, partials, lds);
   } else if (M.val_type == SBLAS_VAL_F32) {
-    rows_typed<float, ITEMS, BLOCK>(w, it, M, partials, lds, wsum);
+    rows_typed<float, ITEMS, BLOCK>(it, M, partials, lds);
   } else {
-    rows_typed<uint16_t, ITEMS, BLOCK>(w, it, M, partials, lds, wsum);
+    rows_typed<uint16_t, ITEMS, BLOCK>(it, M, partials, lds);
   }
 }
 
@@ -350,7 +233,6 @@ __device__ __forceinline__ void batch_loop(const BatchItem *__restrict__ items,
                                            int *__restrict__ ctr) {
   static_assert(BLOCK == 256, "the panel body assumes 256 threads");
   __shared__ double lds[batch_lds<MODE, ITEMS, BLOCK>()];
-  __shared__ double wsum[BLOCK / 64];
   __shared__ int next;
   const int t = threadIdx.x;
   // workgroups are dispatched to the eight XCDs in turn: start on this XCD's
@@ -369,7 +251,7 @@ __device__ __forceinline__ void batch_loop(const BatchItem *__restrict__ items,
       // claim the following item now; its counter round trip overlaps this item
       int claimed = 0;
       if (t == 0) claimed = qbound[q] + atomicAdd(&ctr[q], 1);
-      batch_item<MODE, ITEMS, BLOCK>(w, items, mats, partials, lds, wsum);
+      batch_item<MODE, ITEMS, BLOCK>(w, items, mats, partials, lds);
       if (t == 0) next = claimed;  // last read before this iteration's first barrier
       __syncthreads();
       w = next;
@@ -417,9 +299,10 @@ __global__ __launch_bounds__(256) void k_batch_x32(const BatchX32 *__restrict__ 
   }
 }
 
-// One work item per workgroup, for a launch that shares the GPU with others:
-// the hardware hands out its workgroups as CUs free up, where a persistent
-// launch would hold every CU until its queues drain.  Workgroup b runs on
+// One work item per workgroup, how row blocks run: the hardware hands out
+// workgroups as CUs free up, where a persistent launch would hold every CU
+// until its queues drain (and, at 107 registers against 60, half as many
+// workgroups).  Workgroup b runs on
 // XCD b % 8 and takes item (b % 8) * G/8 + b / 8, so each XCD works through a
 // contiguous run of the list (the grid is a multiple of 8).
 template <int MODE, int ITEMS, int BLOCK>
@@ -429,11 +312,10 @@ __global__ __launch_bounds__(BLOCK) void k_batch_flat(int nitems,
                                                       double *__restrict__ partials) {
   static_assert(BLOCK == 256, "the panel body assumes 256 threads");
   __shared__ double lds[batch_lds<MODE, ITEMS, BLOCK>()];
-  __shared__ double wsum[BLOCK / 64];
   const int per = static_cast<int>(gridDim.x) >> 3;
   const int w = (static_cast<int>(blockIdx.x) & 7) * per + (static_cast<int>(blockIdx.x) >> 3);
   if (w >= nitems) return;
-  batch_item<MODE, ITEMS, BLOCK>(w, items, mats, partials, lds, wsum);
+  batch_item<MODE, ITEMS, BLOCK>(w, items, mats, partials, lds);
 }
 
 // Split rows of all matrices: one thread per row (all its vectors), partials

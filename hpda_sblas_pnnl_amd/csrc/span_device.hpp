@@ -108,6 +108,7 @@ __device__ __forceinline__ void mark_end(Shared<ITEMS> &sh, int e) {
 // they follow every row end.
 template <int ITEMS>
 __device__ __forceinline__ void row_sums(Shared<ITEMS> &sh) {
+  static_assert(sizeof(Shared<ITEMS>) % sizeof(double) == 0, "LDS counted in doubles");
   static_assert(ITEMS == 4 || ITEMS == 8 || ITEMS == 16, "spans of whole mask parts");
   const int t = threadIdx.x;
   const uint32_t m = (sh.ends[(t * ITEMS) >> 5] >> ((t * ITEMS) & 31)) & ((1u << ITEMS) - 1u);
