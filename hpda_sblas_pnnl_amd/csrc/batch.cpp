@@ -316,7 +316,7 @@ int sblas_batch_create(int count, const sblas_batch_item *items, const sblas_opt
                           : kBatchPanelRowsMax;
       int layout = narrow ? kPanelSorted : kPanelRowOrder;
       int st = panel_build(it.val_type, rows, it.m, it.n, it.nnz, it.d_row_ptr, it.d_col,
-                           it.d_val, one, h_rp.data(), want == 3, 1, f, &panel, nullptr, layout);
+                           it.d_val, one, h_rp.data(), want == 3, PanelRule{}, f, &panel, nullptr, layout);
       // panels sized for one round may hold slices too sparse for the form:
       // taller ones while every CU still gets one
       while (st == SBLAS_OK && !panel && narrow && rows < 1024 && !(opts && opts->panel_rows > 0) &&
@@ -324,7 +324,7 @@ int sblas_batch_create(int count, const sblas_batch_item *items, const sblas_opt
         f = PanelFormat{};
         rows = std::min(2 * rows, 1024);
         st = panel_build(it.val_type, rows, it.m, it.n, it.nnz, it.d_row_ptr, it.d_col, it.d_val,
-                         one, h_rp.data(), want == 3, 1, f, &panel, nullptr, layout);
+                         one, h_rp.data(), want == 3, PanelRule{}, f, &panel, nullptr, layout);
       }
       if (st == SBLAS_OK && !panel && narrow && !(opts && opts->panel_rows > 0)) {
         // no launch of its own: the persistent launch's row panels, x in FP64
@@ -333,7 +333,7 @@ int sblas_batch_create(int count, const sblas_batch_item *items, const sblas_opt
         rows = kBatchPanelRowsMax;
         layout = kPanelRowOrder;
         st = panel_build(it.val_type, rows, it.m, it.n, it.nnz, it.d_row_ptr, it.d_col, it.d_val,
-                         one, h_rp.data(), want == 3, 1, f, &panel, nullptr, layout);
+                         one, h_rp.data(), want == 3, PanelRule{}, f, &panel, nullptr, layout);
       }
       // row order with slices beyond 16-bit offsets (the batch kernel reads
       // 16-bit ones only): shorter row panels, down to 192 rows, before
@@ -344,7 +344,7 @@ int sblas_batch_create(int count, const sblas_batch_item *items, const sblas_opt
         f = PanelFormat{};
         rows /= 2;
         st = panel_build(it.val_type, rows, it.m, it.n, it.nnz, it.d_row_ptr, it.d_col, it.d_val,
-                         one, h_rp.data(), want == 3, 1, f, &panel, nullptr, layout);
+                         one, h_rp.data(), want == 3, PanelRule{}, f, &panel, nullptr, layout);
       }
       if (st == SBLAS_OK && panel && layout == kPanelRowOrder && !f.srp)
         panel = false;  // slices beyond 16-bit offsets

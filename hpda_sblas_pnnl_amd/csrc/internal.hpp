@@ -123,7 +123,8 @@ struct SegmentFormat {
   std::vector<void *> buffers;
   int64_t bytes = 0;
 };
-// Builds the format on the device (synchronous); h_vrp receives the virtual
+// Builds the format on the device (synchronous) from rows whose columns
+// ascend; h_vrp receives the virtual
 // row pointers.
 int seg_build(int val_type, int m, int n, int64_t nnz, const int *rp, const int *col,
               const void *val, int P, SegmentFormat &f, std::vector<int> &h_vrp);
@@ -256,18 +257,32 @@ struct PanelFormat {
   std::vector<void *> buffers;
 };
 int panel_rpt(int rows);
-// Rows per row panel so the panels fill whole rounds of resident workgroups.
+// Rows per row panel so the panels fill whole rounds of resident workgroups;
+// *rounds (sorted layout, may be null) = how many.
 int panel_rows_for(int val_type, int m, int device, bool narrow_x = false,
-                   int layout = kPanelRowOrder, int chunks = 1);
+                   int layout = kPanelRowOrder, int chunks = 1, int *rounds = nullptr);
+// *ok = no row's columns descend anywhere (equal neighbours are fine); rp holds
+// m + 1 pointers, rp[m] = nnz.  Synchronous on s.
+int columns_ascend(int m, int64_t nnz, const int *rp, const int *col, hipStream_t s, bool *ok);
+// When the form pays: at least `panels` row panels, each of which on average
+// spans more than `span` column panels, holds `elements` elements and, per row
+// and slice, `per_row` elements (beside the rules of panel_build itself).
+struct PanelRule {
+  int panels = 1;
+  double span = 3.0;
+  int64_t elements = 0;
+  double per_row = 0.0;
+};
 // Builds the format on the device: each execution chunk of `ex` cut into row
 // panels of at most `rows` rows (h_rp: host copy of the row pointers).  With
 // force == false it stops after the per-panel column ranges and sets
-// *chosen = false when the form would not help (few row panels, sparse
-// slices, or rows whose x window is narrow).
+// *chosen = false when the form would not help (the rule, or sparse slices).
+// Also with force, *chosen = false for rows whose columns do not ascend: their
+// elements in a column panel would not be one run.
 // layout kPanelSorted rounds the rows per panel up to a multiple of 64.
 int panel_build(int val_type, int rows, int m, int n, int64_t nnz, const int *rp, const int *col,
                 const void *val, const std::vector<ExecChunk> &ex, const int *h_rp,
-                bool force, int min_panels, PanelFormat &f, bool *chosen, hipStream_t s,
+                bool force, const PanelRule &rule, PanelFormat &f, bool *chosen, hipStream_t s,
                 int layout = kPanelRowOrder);
 // x32_ready: the FP32 copy of x (narrow-x form) is already written.
 int launch_panel_spmv(int val_type, const PanelFormat &f, int m, int n, int xcd_remap,

@@ -913,7 +913,7 @@ int Plan::choose_csr(const std::vector<int> &h_rp) {
     // overrides the auto setting)
     int nxo = opts.narrow_x;
     if (nxo == 0) nxo = env_int("SBLAS_NARROW_X", 0) > 0 ? env_int("SBLAS_NARROW_X", 0) : 2;
-    const bool narrow_x = val_type != SBLAS_VAL_F64 && nxo == 2;
+    bool narrow_x = val_type != SBLAS_VAL_F64 && nxo == 2;
     // slice layout: sorted groups where x is staged in FP32, rows in order
     // otherwise, unless asked (SBLAS_PANEL_LAYOUT overrides the auto setting)
     int lo_opt = opts.panel_layout;
@@ -922,21 +922,61 @@ int Plan::choose_csr(const std::vector<int> &h_rp) {
                        : lo_opt == 1 ? kPanelRowOrder
                        : narrow_x    ? kPanelSorted
                                      : kPanelRowOrder;
-    const int rows =
-        opts.panel_rows > 0
-            ? opts.panel_rows
-            : panel_rows_for(val_type, m, device, narrow_x, layout, static_cast<int>(exec.size()));
+    const int C = static_cast<int>(exec.size());
+    const bool force = opts.variant == 3;
     bool chosen = false;
-    st = panel_build(val_type, rows, m, n, nnz, a0, a1, val, exec, h_rp.data(),
-                     opts.variant == 3, min_panels, panel, &chosen, nullptr, layout);
-    // sorted-layout panels sized for one round may hold slices too sparse
-    // for the form: taller ones (while enough panels remain) before giving up
-    for (int r2 = 2 * rows; st == SBLAS_OK && !chosen && layout == kPanelSorted &&
-                            opts.panel_rows <= 0 && r2 <= 1024 && m / r2 >= min_panels;
-         r2 *= 2) {
+    st = SBLAS_OK;
+    auto build = [&](int rows, const PanelRule &rule, int lay) {
       panel = PanelFormat{};
-      st = panel_build(val_type, r2, m, n, nnz, a0, a1, val, exec, h_rp.data(), false, min_panels,
-                       panel, &chosen, nullptr, layout);
+      return panel_build(val_type, rows, m, n, nnz, a0, a1, val, exec, h_rp.data(), force, rule,
+                         panel, &chosen, nullptr, lay);
+    };
+    // x in FP64, layout and panel height left to the chooser: sorted groups
+    // where they are the better layout, whatever the x window's width.  A lane
+    // owns a row, so long runs of a row in a slice (narrow bands) cost it
+    // nothing, where the row-order body has one thread sum them.  They want
+    // every panel resident at once, a group of 64 rows for each of the four
+    // waves, and 4096 elements a panel.  us, row blocks / row order / sorted:
+    //   FP64 300,000 rows of 27, band 2,000:     25.0 /  23.2 /  21.3
+    //        300,000 of 140, band 3,800:        115.9 / 173.4 /  87.8
+    //        300,000 of 140, band 60,000:       194.8 / 117.4 / 110.3
+    //        512,000 of 27, band 13,000:         60.8 /  39.1 /  36.4
+    //        1,000,000 of 7, band 5,000:         29.0 /  26.9 /  22.8
+    //        1,000,000 of 140, band 5,000:      401.6 / 545.5 / 255.9
+    //   100,000 of 140 (two groups a panel), band 500: 32.7 / 84.2 / 40.6
+    //   500,000 of 4 (2048 elements a panel):          10.3 / 11.9 / 10.1
+    // In several rounds they lose to row order (2,000,000 rows of 140, band
+    // 100,000: 600 / 500; of 27, band 10,000: 116 / 112) unless a row has
+    // more than eight elements in a slice.
+    auto build_sorted64 = [&](double span) -> int {
+      if (opts.variant != 0 || opts.panel_rows > 0 || lo_opt != 0 || stats.max_row > kPanelCols)
+        return SBLAS_OK;
+      int rounds = 1;
+      const int rows = panel_rows_for(val_type, m, device, false, kPanelSorted, C, &rounds);
+      if (rows < 256) return SBLAS_OK;
+      return build(rows, PanelRule{min_panels, span, 4096, rounds > 1 ? 8.0 : 0.0}, kPanelSorted);
+    };
+    if (!narrow_x) st = build_sorted64(0.0);
+    if (st == SBLAS_OK && !chosen) {
+      const int rows = opts.panel_rows > 0
+                           ? opts.panel_rows
+                           : panel_rows_for(val_type, m, device, narrow_x, layout, C);
+      const PanelRule rule{min_panels};
+      st = build(rows, rule, layout);
+      // sorted-layout panels sized for one round may hold slices too sparse
+      // for the form: taller ones (while enough panels remain) before giving up
+      for (int r2 = 2 * rows; st == SBLAS_OK && !chosen && layout == kPanelSorted &&
+                              opts.panel_rows <= 0 && r2 <= 1024 && m / r2 >= min_panels;
+           r2 *= 2)
+        st = build(r2, rule, layout);
+    }
+    if (st == SBLAS_OK && !chosen && narrow_x && narrow_x_asked() == 0) {
+      // narrow bands of narrow values: the forms tried below would mostly read
+      // x in FP64, and so do these panels (BF16, 1,000,000 rows of 140, band
+      // 5,000: 137 us against 296 for row blocks; 300,000 rows of 27, band
+      // 2,000: 15.3 against 18.7)
+      st = build_sorted64(0.0);
+      narrow_x = false;
     }
     if (st == SBLAS_ERR_UNSUPPORTED && opts.variant == 0) {
       // a slice too large for 16-bit offsets: keep the row-block form
@@ -987,6 +1027,10 @@ int Plan::choose_csr(const std::vector<int> &h_rp) {
   }
   if (asked == 6) {
     if (nnz == 0) return SBLAS_OK;  // nothing to segment: row blocks
+    // a row's elements in a segment must be one run: row blocks otherwise
+    bool ascend = true;
+    if ((st = columns_ascend(m, nnz, a0, a1, nullptr, &ascend)) != SBLAS_OK) return st;
+    if (!ascend) return SBLAS_OK;
     if ((st = setup_segments(segments_for(n))) != SBLAS_OK) return st;
     variant = 6;
     return SBLAS_OK;
@@ -1020,7 +1064,9 @@ int Plan::choose_csr(const std::vector<int> &h_rp) {
       return setup_sorted(h_rp.data());
     }
     if (found.variant == 6) {
-      st = setup_segments(segments_for(n));
+      bool ascend = true;
+      if ((st = columns_ascend(m, nnz, a0, a1, nullptr, &ascend)) != SBLAS_OK) return st;
+      st = ascend ? setup_segments(segments_for(n)) : static_cast<int>(SBLAS_ERR_UNSUPPORTED);
       if (st == SBLAS_ERR_ALLOC || st == SBLAS_ERR_UNSUPPORTED) {  // row blocks instead
         clear_error();
         drop_segments();
@@ -1045,7 +1091,11 @@ int Plan::choose_csr(const std::vector<int> &h_rp) {
   // 4 GB.  Row blocks against segments (us): R-MAT with x of 2.4 MB 28.4 /
   // 31.6, 8 MB 100.7 / 93.5, 12 MB 178 / 150, 32 MB 488 / 381.
   const int64_t x_bytes = static_cast<int64_t>(n) * 8;
+  bool ascend = true;
   if (x_bytes > (int64_t{8} << 20) &&
+      (st = columns_ascend(m, nnz, a0, a1, nullptr, &ascend)) != SBLAS_OK)
+    return st;
+  if (x_bytes > (int64_t{8} << 20) && ascend &&
       static_cast<int64_t>(segments_for(n)) * m <= (int64_t{1} << 28)) {
     st = setup_segments(segments_for(n));
     if (st == SBLAS_ERR_ALLOC || st == SBLAS_ERR_UNSUPPORTED) {

@@ -166,6 +166,26 @@ __global__ void k_panel_range(int npanels, PanelInfo *__restrict__ info,
   }
 }
 
+// *diff = columns that descend from one element to the next, less those that
+// do so from one row's last element to the next row's first: 0 when every
+// row's columns ascend.
+__global__ __launch_bounds__(256) void k_column_order(int m, int64_t nnz,
+                                                      const int *__restrict__ rp,
+                                                      const int *__restrict__ col,
+                                                      unsigned long long *__restrict__ diff) {
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
+  const int64_t first = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  long long d = 0;
+  for (int64_t j = first + 1; j < nnz; j += stride) d += col[j] < col[j - 1] ? 1 : 0;
+  for (int64_t r = first; r < m; r += stride) {
+    const int b = rp[r];
+    if (b > 0 && rp[r + 1] > b) d -= col[b] < col[b - 1] ? 1 : 0;
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) d += __shfl_xor(d, off, 64);
+  if ((threadIdx.x & 63) == 0 && d != 0) atomicAdd(diff, static_cast<unsigned long long>(d));
+}
+
 // Element-parallel passes over one row panel's element window: one
 // workgroup per row panel, 1024 elements per step (four consecutive elements
 // per thread).  An element's row comes from a binary search of the panel's
@@ -349,12 +369,31 @@ __global__ void k_narrow_u16(int64_t count, const uint32_t *__restrict__ a,
 
 }  // namespace
 
+int columns_ascend(int m, int64_t nnz, const int *rp, const int *col, hipStream_t s, bool *ok) {
+  *ok = true;
+  if (nnz < 2) return SBLAS_OK;
+  unsigned long long *diff = nullptr, h = 0;
+  SBLAS_HIP_TRY(hipMalloc(&diff, sizeof(h)));
+  hipError_t e = hipMemcpyAsync(diff, &h, sizeof(h), hipMemcpyHostToDevice, s);
+  if (e == hipSuccess) {
+    const int64_t blocks = std::min<int64_t>((nnz + 1023) / 1024, 4096);
+    hipLaunchKernelGGL(k_column_order, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, m, nnz,
+                       rp, col, diff);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) e = hipMemcpyAsync(&h, diff, sizeof(h), hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  (void)hipFree(diff);
+  SBLAS_HIP_TRY(e);
+  *ok = h == 0;
+  return SBLAS_OK;
+}
+
 int panel_build(int val_type, int rows, int m, int n, int64_t nnz, const int *rp, const int *col,
                 const void *val, const std::vector<ExecChunk> &ex, const int *h_rp,
-                bool force, int min_panels, PanelFormat &f, bool *chosen, hipStream_t s,
+                bool force, const PanelRule &rule, PanelFormat &f, bool *chosen, hipStream_t s,
                 int layout) {
   (void)n;
-  (void)m;
   *chosen = false;
   if (rows < 1 || rows > kPanelRowsMax) {
     set_error(SBLAS_ERR_ARGS, "panel format: rows per panel must be in [1, 2048]");
@@ -431,11 +470,12 @@ int panel_build(int val_type, int rows, int m, int n, int64_t nnz, const int *rp
   f.avg_slice = total > 0 ? static_cast<double>(nnz) / total : 0.0;
   // worth it when there are enough row panels to fill the GPU, slices are
   // dense enough that one coalesced pass over a column panel of x costs at
-  // most a quarter of an x line per element, and a row panel's x window
-  // spans more than three column panels (avg_panels * 256 x lines for a
-  // row-parallel block of 2048 elements).  Measured on banded matrices: row
+  // most a quarter of an x line per element, and, in row order, a row panel's
+  // x window spans more than three column panels (avg_panels * 256 x lines for
+  // a row-parallel block of 2048 elements).  Measured on banded matrices: row
   // panels spanning 3.7, 5.2 and 7.7 column panels run 1.2x, 1.4x and 2.1x
-  // faster than row blocks, 2.1 column panels 0.7x.
+  // faster than row blocks, 2.1 column panels 0.7x (a chunk then holds few
+  // rows, and one thread sums each).
   // One workgroup sums a row panel, so a panel holding far more than its
   // share keeps its workgroup running long after the others (the first row
   // panels of an R-MAT matrix hold most of its elements; in the 64-matrix
@@ -445,9 +485,16 @@ int panel_build(int val_type, int rows, int m, int n, int64_t nnz, const int *rp
   for (const int2 &w : hwin) densest = std::max<int64_t>(densest, w.y - w.x);
   const bool balanced =
       densest <= std::max<int64_t>(65536, 4 * nnz / std::max(f.npanels, 1));
-  const bool helps = f.npanels >= min_panels && f.avg_slice >= 1024.0 &&
-                     f.avg_panels_per_row_panel > 3.0 && balanced;
-  if (!force && !helps) {
+  const bool helps = f.npanels >= rule.panels && f.avg_slice >= 1024.0 &&
+                     f.avg_panels_per_row_panel > rule.span &&
+                     nnz >= rule.elements * f.npanels && f.avg_slice >= rule.per_row * R &&
+                     balanced;
+  bool ascend = true;
+  if (force || helps) {
+    const int st = columns_ascend(m, nnz, rp, col, s, &ascend);
+    if (st != SBLAS_OK) return st;
+  }
+  if ((!force && !helps) || !ascend) {
     for (void *p : f.buffers) (void)hipFree(p);
     f.buffers.clear();
     f.npanels = 0;
@@ -785,7 +832,8 @@ int sorted_occupancy(int val_type, bool narrow_x, int rpt) {
 }
 }  // namespace
 
-int panel_rows_for(int val_type, int m, int device, bool narrow_x, int layout, int chunks) {
+int panel_rows_for(int val_type, int m, int device, bool narrow_x, int layout, int chunks,
+                   int *rounds) {
   int cus = 256, per_cu = 0;
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
   const void *fn =
@@ -826,7 +874,9 @@ int panel_rows_for(int val_type, int m, int device, bool narrow_x, int layout, i
         if (room < 1) continue;
         int64_t R = (m + room - 1) / room;
         R = (R + 63) / 64 * 64;
-        if (R <= 256 * rpt) return static_cast<int>(std::max<int64_t>(R, 64));
+        if (R > 256 * rpt) continue;
+        if (rounds) *rounds = static_cast<int>(k);
+        return static_cast<int>(std::max<int64_t>(R, 64));
       }
     }
   }
