@@ -39,6 +39,7 @@ HIP_SOURCES = [
     "stream.cpp",
     "staging.cpp",
     "plan.cpp",
+    "direct.cpp",
     "dropin.cpp",
     "partition.cpp",
 ]

@@ -2,7 +2,8 @@
 // on one MI355X.
 //
 // Each call is synchronous and stateless like the reference's: the caller's
-// host arrays are uploaded, a plan is built with the entry point's partition
+// host arrays are uploaded, a plan is built (CSR matrices that with their
+// vectors take up to 64 MB go without one, direct.cpp) with the entry point's partition
 // rule at the configured chunk count (ngpu must be 1; chunks come from
 // SBLAS_CHUNKS, default 1), the kernel runs on a private stream, split rows
 // are merged on the device and y is copied back.  spmv_ret holds the times of
@@ -21,6 +22,7 @@
 #include <limits>
 #include <vector>
 
+#include "direct.hpp"
 #include "host_util.hpp"
 #include "plan.hpp"
 
@@ -83,6 +85,13 @@ spmv_ret run_format(int format, int m, int n, int nnz, const double *alpha, cons
   if (!guard.ok) {
     set_error(SBLAS_ERR_NO_DEVICE, "no HIP device");
     return nan_ret();
+  }
+  if (format == SBLAS_FMT_CSR && !sparse_x && q == 1) {
+    bool handled = false;
+    const int st = direct_csr(env_int("SBLAS_DEVICE", 0), m, n, nnz, *alpha, val, a0, a1, x,
+                              *beta, y, kernel, part_mode, ret, handled);
+    if (st != SBLAS_OK) return nan_ret();
+    if (handled) return ret;
   }
   hipStream_t s = nullptr;
   if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) {

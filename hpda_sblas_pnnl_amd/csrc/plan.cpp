@@ -578,6 +578,34 @@ int Plan::setup_tiles() {
   return SBLAS_OK;
 }
 
+void csr5_host_format(int m, int64_t nnz, int sg, const int *h_rp, Csr5Host &h) {
+  const int64_t T = 64LL * sg;
+  h.tiles = static_cast<int>((nnz + T - 1) / T);
+  std::vector<int> nzidx(static_cast<size_t>(std::max(m, 1)), -1);
+  for (int r = 0; r < m; r++) {
+    if (h_rp[r + 1] > h_rp[r]) {
+      nzidx[r] = static_cast<int>(h.rows_nz.size());
+      h.rows_nz.push_back(r);
+    } else {
+      h.empty.push_back(r);
+    }
+  }
+  h.tile_nz.assign(static_cast<size_t>(std::max(h.tiles, 1)), 0);
+  h.flags.assign(static_cast<size_t>(std::max(h.tiles, 1)) * 64, 0);
+  int r = 0;
+  for (int p = 0; p < h.tiles; p++) {
+    const int64_t e = static_cast<int64_t>(p) * T;
+    while (h_rp[r + 1] <= e) r++;
+    h.tile_nz[p] = static_cast<uint32_t>(nzidx[r]) | (h_rp[r] == e ? 0x80000000u : 0u);
+  }
+  for (int q : h.rows_nz) {
+    const int64_t e = h_rp[q];
+    const int64_t o = e % T;
+    if (o == 0) continue;  // tile start: bit 31 of the tile word
+    h.flags[static_cast<size_t>(e / T) * 64 + static_cast<size_t>(o / sg)] |= 1u << (o % sg);
+  }
+}
+
 // CSR5-style format: tiles of 64 lanes x sigma elements; per tile the index
 // of its first row among the non-empty rows (bit 31: the tile begins at a
 // row start); per lane a word of row-start bits; the element arrays copied
@@ -590,30 +618,11 @@ int Plan::setup_csr5(const std::vector<int> &h_rp) {
   }
   sigma = sg;
   const int64_t T = 64LL * sg;
-  tiles = static_cast<int>((nnz + T - 1) / T);
-  std::vector<int> rows_nz, empty, nzidx(static_cast<size_t>(std::max(m, 1)), -1);
-  for (int r = 0; r < m; r++) {
-    if (h_rp[r + 1] > h_rp[r]) {
-      nzidx[r] = static_cast<int>(rows_nz.size());
-      rows_nz.push_back(r);
-    } else {
-      empty.push_back(r);
-    }
-  }
-  std::vector<uint32_t> tile_nz(static_cast<size_t>(std::max(tiles, 1)), 0);
-  std::vector<uint32_t> flags(static_cast<size_t>(std::max(tiles, 1)) * 64, 0);
-  int r = 0;
-  for (int p = 0; p < tiles; p++) {
-    const int64_t e = static_cast<int64_t>(p) * T;
-    while (h_rp[r + 1] <= e) r++;
-    tile_nz[p] = static_cast<uint32_t>(nzidx[r]) | (h_rp[r] == e ? 0x80000000u : 0u);
-  }
-  for (int q : rows_nz) {
-    const int64_t e = h_rp[q];
-    const int64_t o = e % T;
-    if (o == 0) continue;  // tile start: bit 31 of the tile word
-    flags[static_cast<size_t>(e / T) * 64 + static_cast<size_t>(o / sg)] |= 1u << (o % sg);
-  }
+  Csr5Host h;
+  csr5_host_format(m, nnz, sg, h_rp.data(), h);
+  tiles = h.tiles;
+  const std::vector<int> &rows_nz = h.rows_nz, &empty = h.empty;
+  const std::vector<uint32_t> &tile_nz = h.tile_nz, &flags = h.flags;
   c5_empty = static_cast<int>(empty.size());
   int st;
   if ((st = upload(*this, &d_c5_tile_nz, tile_nz)) != SBLAS_OK) return st;

@@ -17,6 +17,14 @@ int autotune_subwave(const RowStats &s);
 int autotune_sigma(int64_t nnz, int m);
 std::vector<RowBlock> build_row_blocks(const std::vector<ExecChunk> &ex, const int *rp,
                                        int cap);
+// Host part of the CSR5-style format (plan.cpp, sblas_csr5.hip): tiles of 64
+// lanes x sigma elements.
+struct Csr5Host {
+  int tiles = 0;
+  std::vector<int> rows_nz, empty;      // rows with and without elements
+  std::vector<uint32_t> tile_nz, flags;  // per tile, per lane
+};
+void csr5_host_format(int m, int64_t nnz, int sigma, const int *h_rp, Csr5Host &h);
 const char *last_message();
 // Vector-kernel (sub-wave) launch shape over execution chunks; dev receives
 // one DevChunk per chunk.

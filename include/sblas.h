@@ -4,7 +4,9 @@
  * Four layers:
  *   1. Drop-in entry points with the reference's names and argument lists
  *      (include/spmv_kernel.h:211-296 of the reference).  Host pointers,
- *      synchronous, y = alpha*A*x + beta*y, ngpu must be 1.
+ *      synchronous, y = alpha*A*x + beta*y, ngpu must be 1.  From the first
+ *      call on, the library keeps a stream, up to 64 MB of device memory and
+ *      1 MB of pinned memory per device for calls on CSR matrices that fit.
  *   2. Partition API: the reference's chunking rules evaluated at any chunk
  *      count C, returning one descriptor per chunk.
  *   3. Plan API on device-resident arrays (the analogue of the reference's
