@@ -221,6 +221,38 @@ int upload(Plan &p, T **dst, const std::vector<T> &src) {
 
 }  // namespace
 
+namespace {
+
+// Small host arrays uploaded together: one allocation and one transfer (a
+// synchronous transfer of its own costs each about 15 us).
+class Uploads {
+ public:
+  template <typename T>
+  void add(T **dst, const std::vector<T> &src) {
+    const size_t at = bytes_.size(), n = sizeof(T) * src.size();
+    bytes_.resize((at + std::max<size_t>(n, 1) + 255) & ~size_t{255});
+    if (n) std::memcpy(bytes_.data() + at, src.data(), n);
+    places_.emplace_back(reinterpret_cast<void **>(dst), at);
+  }
+  int send(Plan &p) {
+    char *d = static_cast<char *>(p.dev_alloc(bytes_.size()));
+    if (!d) {
+      set_error(SBLAS_ERR_ALLOC, "plan: device allocation failed");
+      return SBLAS_ERR_ALLOC;
+    }
+    if (!bytes_.empty())
+      SBLAS_HIP_TRY(hipMemcpy(d, bytes_.data(), bytes_.size(), hipMemcpyHostToDevice));
+    for (const auto &q : places_) *q.first = d + q.second;
+    return SBLAS_OK;
+  }
+
+ private:
+  std::vector<char> bytes_;
+  std::vector<std::pair<void **, size_t>> places_;
+};
+
+}  // namespace
+
 int Plan::build_csr_chunks(const int *h_rp) {
   const int C = chunks;
   const int inz = static_cast<int>(nnz);
@@ -265,9 +297,11 @@ int Plan::build_csr_chunks(const int *h_rp) {
   ngroups = static_cast<int>(mrows.size());
   split_rows = ngroups;
   int st;
-  if ((st = upload(*this, &d_mrows, mrows)) != SBLAS_OK) return st;
-  if ((st = upload(*this, &d_mptr, mptr)) != SBLAS_OK) return st;
-  if ((st = upload(*this, &d_mslots, mslots)) != SBLAS_OK) return st;
+  Uploads up;
+  up.add(&d_mrows, mrows);
+  up.add(&d_mptr, mptr);
+  up.add(&d_mslots, mslots);
+  if ((st = up.send(*this)) != SBLAS_OK) return st;
   d_partials = static_cast<double *>(dev_alloc(sizeof(double) * 2 * exec.size() * max_k));
   if (!d_partials) {
     set_error(SBLAS_ERR_ALLOC, "plan: partials allocation failed");
@@ -369,16 +403,18 @@ int Plan::setup_stream(const int *h_rp) {
   sl.xcd_remap = remap ? 1 : 0;
   sl.grid = remap ? ((sl.nblocks + 7) / 8) * 8 : sl.nblocks;
   int st;
-  if ((st = upload(*this, &d_rblocks, rblocks)) != SBLAS_OK) return st;
+  Uploads up;
+  up.add(&d_rblocks, rblocks);
   std::vector<ExecChunk> as_chunks;
   as_chunks.reserve(rblocks.size());
   for (const RowBlock &b : rblocks) as_chunks.push_back(ExecChunk{b.lo, b.hi, b.row_begin, b.row_end});
   std::vector<int> mrows, mptr, mslots;
   merge_lists(as_chunks, h_rp, mrows, mptr, mslots);
   bgroups = static_cast<int>(mrows.size());
-  if ((st = upload(*this, &d_bmrows, mrows)) != SBLAS_OK) return st;
-  if ((st = upload(*this, &d_bmptr, mptr)) != SBLAS_OK) return st;
-  if ((st = upload(*this, &d_bmslots, mslots)) != SBLAS_OK) return st;
+  up.add(&d_bmrows, mrows);
+  up.add(&d_bmptr, mptr);
+  up.add(&d_bmslots, mslots);
+  if ((st = up.send(*this)) != SBLAS_OK) return st;
   // 2 slots per block, max_k values per slot (multi-RHS blocks use the same list)
   d_bpartials = static_cast<double *>(
       dev_alloc(sizeof(double) * 2 * max_k * std::max<size_t>(rblocks.size(), 1)));
@@ -386,6 +422,47 @@ int Plan::setup_stream(const int *h_rp) {
     set_error(SBLAS_ERR_ALLOC, "plan: partials allocation failed");
     return SBLAS_ERR_ALLOC;
   }
+  return setup_short_blocks(h_rp);
+}
+
+// Row blocks of 512 elements for products of 8 or 16 vectors over matrices of
+// at most two 2048-element blocks a CU: k/2 lanes share an element there, so a
+// long block keeps its few groups busy for 32 or 64 elements each while most
+// CUs idle.  k = 8 / 16, us with blocks of 2048 -> 512: R-MAT 9,537 rows (47
+// blocks) 13.6 / 21.8 -> 10.2 / 14.0, 30,000 rows (186) 16.2 / 25.1 -> 11.9 /
+// 15.6; 10,000 rows of 7 (35) 9.5 / 15.4 -> 4.7 / 6.0; 100,000 rows of 10 (491)
+// 10.7 / 14.4 -> 9.1 / 12.1; above, equal or slower (power law, 60,000 rows, 516
+// blocks: 15.0 / 20.0 -> 17.1 / 21.5; R-MAT 300,000 rows 63 / 83 -> 76 / 93).
+int Plan::setup_short_blocks(const int *h_rp) {
+  slk = StreamLaunch{};
+  int cus = 256;
+  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
+  if (opts.items > 0 || sl.nblocks > 2 * std::max(cus, 1)) return SBLAS_OK;
+  const int items = 2;
+  const std::vector<RowBlock> kb = build_row_blocks(exec, h_rp, kStreamBlock * items);
+  std::vector<ExecChunk> as_chunks;
+  as_chunks.reserve(kb.size());
+  for (const RowBlock &b : kb) as_chunks.push_back(ExecChunk{b.lo, b.hi, b.row_begin, b.row_end});
+  std::vector<int> mrows, mptr, mslots;
+  merge_lists(as_chunks, h_rp, mrows, mptr, mslots);
+  kgroups = static_cast<int>(mrows.size());
+  int st;
+  Uploads up;
+  up.add(&d_kblocks, kb);
+  up.add(&d_kmrows, mrows);
+  up.add(&d_kmptr, mptr);
+  up.add(&d_kmslots, mslots);
+  if ((st = up.send(*this)) != SBLAS_OK) return st;
+  d_kpartials = static_cast<double *>(
+      dev_alloc(sizeof(double) * 2 * max_k * std::max<size_t>(kb.size(), 1)));
+  if (!d_kpartials) {
+    set_error(SBLAS_ERR_ALLOC, "plan: partials allocation failed");
+    return SBLAS_ERR_ALLOC;
+  }
+  slk = sl;
+  slk.items = items;
+  slk.nblocks = static_cast<int>(kb.size());
+  slk.grid = slk.xcd_remap ? ((slk.nblocks + 7) / 8) * 8 : slk.nblocks;
   return SBLAS_OK;
 }
 
@@ -512,14 +589,14 @@ int Plan::run_spmm(int k, double alpha, const double *X, double beta, double *Y,
   if (variant >= 2 && k > 1 && streams.empty()) {
     hipEvent_t *te = timing_slot();
     if (te) SBLAS_HIP_TRY(hipEventRecord(te[0], s));
-    st = launch_csr_blocks_mrhs(val_type, k, sl, d_rblocks, a0, a1, val, X, Y, alpha, beta,
-                                d_bpartials, s);
+    const bool own = short_blocks(k);
+    st = launch_csr_blocks_mrhs(val_type, k, own ? slk : sl, own ? d_kblocks : d_rblocks, a0, a1,
+                                val, X, Y, alpha, beta, own ? d_kpartials : d_bpartials, s);
     if (st != SBLAS_OK) return st;
     if (te) SBLAS_HIP_TRY(hipEventRecord(te[1], s));
     launches++;
-    if (bgroups > 0 && merge_enabled) {
-      st = launch_merge(d_bmrows, d_bmptr, d_bmslots, bgroups, d_bpartials, k, Y, alpha, beta, s);
-      if (st != SBLAS_OK) return st;
+    if (has_merge(k) && merge_enabled) {
+      if ((st = run_merge(k, alpha, beta, Y, s)) != SBLAS_OK) return st;
       launches++;
     }
     return SBLAS_OK;
@@ -1163,7 +1240,8 @@ bool Plan::has_merge(int k) const {
   if (variant == 6 && k == 1 && streams.empty()) return false;  // merges run inside the product
   if (variant == 3 && k == 1 && streams.empty()) return pgroups > 0;
   if (variant == 4 && k == 1 && streams.empty()) return sgroups > 0;
-  if (variant >= 2 && streams.empty()) return bgroups > 0;  // row blocks (any k)
+  if (variant >= 2 && streams.empty())  // row blocks (any k)
+    return short_blocks(k) ? kgroups > 0 : bgroups > 0;
   return ngroups > 0;
 }
 
@@ -1177,6 +1255,10 @@ int Plan::run_merge(int k, double alpha, double beta, double *Y, hipStream_t s) 
                        : SBLAS_OK;
   if (variant == 4 && k == 1 && streams.empty())
     return sgroups > 0 ? launch_merge(d_smrows, d_smptr, d_smslots, sgroups, sorted.partials, 1, Y,
+                                      alpha, beta, s)
+                       : SBLAS_OK;
+  if (variant >= 2 && streams.empty() && short_blocks(k))
+    return kgroups > 0 ? launch_merge(d_kmrows, d_kmptr, d_kmslots, kgroups, d_kpartials, k, Y,
                                       alpha, beta, s)
                        : SBLAS_OK;
   if (variant >= 2 && streams.empty())

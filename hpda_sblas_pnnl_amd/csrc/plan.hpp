@@ -75,6 +75,14 @@ struct Plan {
   int *d_bmrows = nullptr, *d_bmptr = nullptr, *d_bmslots = nullptr;
   int bgroups = 0;
   double *d_bpartials = nullptr;
+  // shorter row blocks for products of many vectors over small matrices
+  // (setup_short_blocks); grid 0: the row blocks above serve them
+  StreamLaunch slk{};
+  RowBlock *d_kblocks = nullptr;
+  int *d_kmrows = nullptr, *d_kmptr = nullptr, *d_kmslots = nullptr;
+  int kgroups = 0;
+  double *d_kpartials = nullptr;
+
   // segmented tiles (COO / merge path / CSR5)
   int tiles = 0;
   int sigma = 0;
@@ -136,6 +144,14 @@ struct Plan {
   int build_csr_chunks(const int *h_rp);
   int setup_vector(const int *h_rp);
   int setup_stream(const int *h_rp);
+  int setup_short_blocks(const int *h_rp);
+  // With 8 vectors they must not bring a merge launch that the long blocks do
+  // without, unless those are fewer still (power law, 20,000 rows, 171 blocks:
+  // 9.4 us with long blocks, 9.7 with short ones).
+  bool short_blocks(int k) const {
+    return slk.grid > 0 &&
+           (k >= 16 || (k == 8 && (kgroups == 0 || bgroups > 0 || sl.nblocks <= 128)));
+  }
   bool merge_enabled = true;          // false: caller launches run_merge itself
   bool uses_tiles(int k) const;
   // carries left for the ordered fix-up: one per tile, or one per workgroup

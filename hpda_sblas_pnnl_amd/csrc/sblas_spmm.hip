@@ -254,6 +254,8 @@ int launch_spmm_typed(int k, const StreamLaunch &L, const RowBlock *blocks, cons
                       double beta, double *partials, hipStream_t s) {
   if (L.items == 16)
     return launch_spmm_items<VT, 16>(k, L, blocks, rp, col, val, X, Y, alpha, beta, partials, s);
+  if (L.items == 2)
+    return launch_spmm_items<VT, 2>(k, L, blocks, rp, col, val, X, Y, alpha, beta, partials, s);
   return launch_spmm_items<VT, 8>(k, L, blocks, rp, col, val, X, Y, alpha, beta, partials, s);
 }
 
@@ -264,8 +266,8 @@ int launch_csr_blocks_mrhs(int val_type, int k, const StreamLaunch &L, const Row
                            double *Y, double alpha, double beta, double *partials,
                            hipStream_t s) {
   if (L.grid <= 0) return SBLAS_OK;
-  if (L.items != 8 && L.items != 16) {
-    set_error(SBLAS_ERR_ARGS, "spmm kernel: items per thread must be 8 or 16");
+  if (L.items != 2 && L.items != 8 && L.items != 16) {
+    set_error(SBLAS_ERR_ARGS, "spmm kernel: items per thread must be 2, 8 or 16");
     return SBLAS_ERR_ARGS;
   }
   switch (val_type) {
