@@ -1031,16 +1031,17 @@ int Plan::choose_csr(const std::vector<int> &h_rp) {
     //        1,000,000 of 140, band 5,000:      401.6 / 545.5 / 255.9
     //   100,000 of 140 (two groups a panel), band 500: 32.7 / 84.2 / 40.6
     //   500,000 of 4 (2048 elements a panel):          10.3 / 11.9 / 10.1
-    // In several rounds they lose to row order (2,000,000 rows of 140, band
-    // 100,000: 600 / 500; of 27, band 10,000: 116 / 112) unless a row has
-    // more than eight elements in a slice.
+    // In several rounds they lose to row order unless a row has more than 18
+    // elements in a slice.  2,000,000 rows, row order / sorted, by that number:
+    //   2.7: 500 / 600 (140 a row)   6.7: 116 / 125 (30)   10.5: 211 / 223 (60)
+    //   13.1: 394 / 424   17.9: 410 / 418   22.9: 550 / 415   28.2: 597 / 414 (120)
     auto build_sorted64 = [&](double span) -> int {
       if (opts.variant != 0 || opts.panel_rows > 0 || lo_opt != 0 || stats.max_row > kPanelCols)
         return SBLAS_OK;
       int rounds = 1;
       const int rows = panel_rows_for(val_type, m, device, false, kPanelSorted, C, &rounds);
       if (rows < 256) return SBLAS_OK;
-      return build(rows, PanelRule{min_panels, span, 4096, rounds > 1 ? 8.0 : 0.0}, kPanelSorted);
+      return build(rows, PanelRule{min_panels, span, 4096, rounds > 1 ? 18.0 : 0.0}, kPanelSorted);
     };
     if (!narrow_x) st = build_sorted64(0.0);
     if (st == SBLAS_OK && !chosen) {
