@@ -30,6 +30,7 @@ HIP_SOURCES = [
     "sblas_csr5.hip",
     "sblas_batch.hip",
     "sblas_panel.hip",
+    "sblas_panel_spmm.hip",
     "sblas_sorted.hip",
     "sblas_segment.hip",
     "sblas_convert.hip",

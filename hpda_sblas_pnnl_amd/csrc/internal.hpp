@@ -245,7 +245,7 @@ struct PanelFormat {
   int groups = 0;
   uint16_t *perm = nullptr;
   uint32_t *goff = nullptr;
-  double *partials = nullptr;   // 2 slots per row panel
+  double *partials = nullptr;   // 2 slots per row panel, up to kPanelVectors each
   // narrow-x form (FP32 / BF16 values): FP32 copy of x written before each
   // launch, padded with zeros to whole column panels; nullptr: FP64 x
   float *x32 = nullptr;
@@ -288,6 +288,13 @@ int panel_build(int val_type, int rows, int m, int n, int64_t nnz, const int *rp
 int launch_panel_spmv(int val_type, const PanelFormat &f, int m, int n, int xcd_remap,
                       const double *x, double *y, double alpha, double beta, hipStream_t s,
                       bool x32_ready = false);
+
+// Products of two and four vectors over column panels in sorted groups
+// (sblas_panel_spmm.hip): vectors a pass, 0 where row blocks take the product.
+int panel_spmm_vectors(const PanelFormat &f, int k);
+int launch_panel_spmm(int val_type, const PanelFormat &f, int n, int k, int each, int xcd_remap,
+                      const double *X, double *Y, double alpha, double beta, hipStream_t s);
+constexpr int kPanelVectors = 4;  // vectors in a partial slot of a row panel
 
 // batched matrices (sblas_batch.hip)
 struct BatchMatrix {

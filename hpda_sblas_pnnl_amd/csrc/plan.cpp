@@ -586,6 +586,19 @@ int Plan::run_spmm(int k, double alpha, const double *X, double beta, double *Y,
     }
     return SBLAS_OK;
   }
+  if (const int each = panel_vectors(k)) {
+    hipEvent_t *te = timing_slot();
+    if (te) SBLAS_HIP_TRY(hipEventRecord(te[0], s));
+    st = launch_panel_spmm(val_type, panel, n, k, each, vl.xcd_remap, X, Y, alpha, beta, s);
+    if (st != SBLAS_OK) return st;
+    if (te) SBLAS_HIP_TRY(hipEventRecord(te[1], s));
+    launches += k / each;
+    if (has_merge(k) && merge_enabled) {
+      if ((st = run_merge(k, alpha, beta, Y, s)) != SBLAS_OK) return st;
+      launches++;
+    }
+    return SBLAS_OK;
+  }
   if (variant >= 2 && k > 1 && streams.empty()) {
     hipEvent_t *te = timing_slot();
     if (te) SBLAS_HIP_TRY(hipEventRecord(te[0], s));
@@ -1239,7 +1252,7 @@ bool Plan::uses_tiles(int k) const {
 bool Plan::has_merge(int k) const {
   if (uses_tiles(k)) return tiles > 0;
   if (variant == 6 && k == 1 && streams.empty()) return false;  // merges run inside the product
-  if (variant == 3 && k == 1 && streams.empty()) return pgroups > 0;
+  if ((variant == 3 && k == 1 && streams.empty()) || panel_vectors(k)) return pgroups > 0;
   if (variant == 4 && k == 1 && streams.empty()) return sgroups > 0;
   if (variant >= 2 && streams.empty())  // row blocks (any k)
     return short_blocks(k) ? kgroups > 0 : bgroups > 0;
@@ -1250,8 +1263,8 @@ int Plan::run_merge(int k, double alpha, double beta, double *Y, hipStream_t s) 
   if (variant == 6 && k == 1 && streams.empty()) return SBLAS_OK;
   if (uses_tiles(k))
     return tiles > 0 ? launch_tile_fixup(carry_count(), d_carry, Y, alpha, beta, s) : SBLAS_OK;
-  if (variant == 3 && k == 1 && streams.empty())
-    return pgroups > 0 ? launch_merge(d_pmrows, d_pmptr, d_pmslots, pgroups, panel.partials, 1, Y,
+  if ((variant == 3 && k == 1 && streams.empty()) || panel_vectors(k))
+    return pgroups > 0 ? launch_merge(d_pmrows, d_pmptr, d_pmslots, pgroups, panel.partials, k, Y,
                                       alpha, beta, s)
                        : SBLAS_OK;
   if (variant == 4 && k == 1 && streams.empty())

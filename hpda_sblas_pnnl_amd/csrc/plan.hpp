@@ -152,6 +152,11 @@ struct Plan {
     return slk.grid > 0 &&
            (k >= 16 || (k == 8 && (kgroups == 0 || bgroups > 0 || sl.nblocks <= 128)));
   }
+  // vectors a pass of a multi-vector product over the plan's column panels,
+  // 0 where it takes the row blocks
+  int panel_vectors(int k) const {
+    return variant == 3 && k > 1 && streams.empty() ? panel_spmm_vectors(panel, k) : 0;
+  }
   bool merge_enabled = true;          // false: caller launches run_merge itself
   bool uses_tiles(int k) const;
   // carries left for the ordered fix-up: one per tile, or one per workgroup

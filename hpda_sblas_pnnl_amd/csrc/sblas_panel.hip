@@ -518,7 +518,7 @@ int panel_build(int val_type, int rows, int m, int n, int64_t nnz, const int *rp
   int64_t *snnz = static_cast<int64_t *>(alloc(sizeof(int64_t) * (ns + 1)));
   f.slice_off = static_cast<int64_t *>(alloc(sizeof(int64_t) * (ns + 1)));
   int *overflow = static_cast<int *>(alloc(sizeof(int)));
-  f.partials = static_cast<double *>(alloc(sizeof(double) * 2 * np));
+  f.partials = static_cast<double *>(alloc(sizeof(double) * 2 * kPanelVectors * np));
   if (!cnt || (sorted ? (!f.perm || !rank || !f.goff) : !f.srp32) || !snnz || !f.slice_off ||
       !overflow || !f.partials) {
     set_error(SBLAS_ERR_ALLOC, "panel format: allocation failed");
