@@ -69,7 +69,10 @@ struct CallContext {
       dev_bytes = 0;
       const size_t want = (bytes + (size_t{1} << 20) - 1) >> 20 << 20;
       void *p = nullptr;
-      if (hipMalloc(&p, want) != hipSuccess) return false;
+      if (hipMalloc(&p, want) != hipSuccess) {
+        (void)hipGetLastError();  // the plan path's launches must not find it
+        return false;
+      }
       dev = static_cast<char *>(p);
       dev_bytes = want;
     }

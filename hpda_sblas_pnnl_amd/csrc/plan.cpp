@@ -942,6 +942,94 @@ int Plan::narrow_x_asked() const {
   return opts.narrow_x != 0 ? opts.narrow_x : std::max(env_int("SBLAS_NARROW_X", 0), 0);
 }
 
+// Whether narrow values in row blocks (or segments; 0: not among the forms)
+// gather x from an FP32 copy, by the trial's times in ms.  A matrix had the copy
+// where row blocks that sum rows by lane groups beat the column-sorted form; a
+// faster row-block kernel must not take FP64 x from the matrices that had it,
+// so those times are put back: rows * (0.975 + 0.104 where x fits in an XCD's
+// L2, less beyond) + 1.8 us for each unit of the rows' CV above 4 + 0.25 us,
+// within 9 % on 28 of 29 matrices (banded, power law, R-MAT; 1 to 43 M elements,
+// rows 8 to 240 us).  By these estimates the matrices that had the copy lie
+// below 0.94 of the column-sorted form, those with x in FP64 above 0.99, but for
+// two R-MAT ties (1.01 and 1.00) that now read x in FP64.
+bool Plan::rows_take_x32(float rows_ms, float seg_ms, float sorted_ms) const {
+  const double share = std::min(1.0, static_cast<double>(4 << 20) / (8.0 * std::max(n, 1)));
+  double t = rows_ms * (0.975 + 0.104 * share) + 1.8e-3 * std::max(0.0, stats.cv - 4.0) + 2.5e-4;
+  if (seg_ms > 0.f) t = std::min(t, 1.03 * static_cast<double>(seg_ms));
+  return t < 0.96 * static_cast<double>(sorted_ms);
+}
+
+// x in FP64, layout and panel height left to the chooser: sorted groups
+// where they are the better layout, whatever the x window's width.  A lane
+// owns a row, so long runs of a row in a slice (narrow bands) cost it
+// nothing, where the row-order body has one thread sum them.  They want
+// every panel resident at once, a group of 64 rows for each of the four
+// waves, and 4096 elements a panel.  us, row blocks / row order / sorted:
+//   FP64 300,000 rows of 27, band 2,000:     25.0 /  23.2 /  21.3
+//        300,000 of 140, band 3,800:        115.9 / 173.4 /  87.8
+//        300,000 of 140, band 60,000:       194.8 / 117.4 / 110.3
+//        512,000 of 27, band 13,000:         60.8 /  39.1 /  36.4
+//        1,000,000 of 7, band 5,000:         29.0 /  26.9 /  22.8
+//        1,000,000 of 140, band 5,000:      401.6 / 545.5 / 255.9
+//   100,000 of 140 (two groups a panel), band 500: 32.7 / 84.2 / 40.6
+//   500,000 of 4 (2048 elements a panel):          10.3 / 11.9 / 10.1
+// In several rounds they lose to row order unless a row has more than 18
+// elements in a slice.  2,000,000 rows, row order / sorted, by that number:
+//   2.7: 500 / 600 (140 a row)   6.7: 116 / 125 (30)   10.5: 211 / 223 (60)
+//   13.1: 394 / 424   17.9: 410 / 418   22.9: 550 / 415   28.2: 597 / 414 (120)
+int Plan::build_sorted64(const std::vector<int> &h_rp, bool *chosen) {
+  *chosen = false;
+  if (opts.variant != 0 || opts.panel_rows > 0 || opts.panel_layout != 0 ||
+      env_int("SBLAS_PANEL_LAYOUT", 0) != 0 || stats.max_row > kPanelCols)
+    return SBLAS_OK;
+  int cus = 256, rounds = 1;
+  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
+  const int rows = panel_rows_for(val_type, m, device, false, kPanelSorted,
+                                  static_cast<int>(exec.size()), &rounds);
+  if (rows < 256) return SBLAS_OK;
+  panel = PanelFormat{};
+  return panel_build(val_type, rows, m, n, nnz, a0, a1, val, exec, h_rp.data(), false,
+                     PanelRule{2 * std::max(cus, 1), 0.0, 4096, rounds > 1 ? 18.0 : 0.0}, panel,
+                     chosen, nullptr, kPanelSorted);
+}
+
+// The plan's products run over its column panels from now on.
+int Plan::use_panels(const std::vector<int> &h_rp) {
+  kernel = SBLAS_KERNEL_VECTOR;
+  variant = 3;
+  int remap = opts.xcd_remap;
+  if (remap < 0) remap = env_int("SBLAS_XCD_REMAP", 1);
+  vl.xcd_remap = remap ? 1 : 0;
+  // rows cut by chunk edges: partials of their panels, merged in panel order
+  std::vector<int> mrows, mptr, mslots;
+  merge_lists(panel.hpanels, h_rp.data(), mrows, mptr, mslots);
+  pgroups = static_cast<int>(mrows.size());
+  int st;
+  if ((st = upload(*this, &d_pmrows, mrows)) != SBLAS_OK) return st;
+  if ((st = upload(*this, &d_pmptr, mptr)) != SBLAS_OK) return st;
+  return upload(*this, &d_pmslots, mslots);
+}
+
+// Narrow values whose row blocks would read x in FP64, on narrow bands: panels
+// in sorted groups with x in FP64 in their place (FP32, 850,000 rows of 37, band
+// 2,100: 81 -> 50 us; 794,000 of 28, band 2,000: 61 -> 38; 1,074,000 of 8, band
+// 2,700: 36 -> 26).  Where row blocks gather from an FP32 copy of x they stay:
+// the results are then those of that copy.
+int Plan::band_panels(const std::vector<int> &h_rp, bool *chosen) {
+  *chosen = false;
+  if (stats.max_row > 8192) return SBLAS_OK;
+  int st = build_sorted64(h_rp, chosen);
+  if (st == SBLAS_ERR_UNSUPPORTED || st == SBLAS_ERR_ALLOC) {
+    for (void *p : panel.buffers) (void)hipFree(p);
+    panel = PanelFormat{};
+    *chosen = false;
+    clear_error();
+    (void)hipGetLastError();
+    return SBLAS_OK;
+  }
+  return st;
+}
+
 // Kernel choice and launch set-up for a CSR matrix whose row pointer is h_rp
 // (the caller's CSR, or the row-major form built from a CSC matrix).
 //
@@ -1030,33 +1118,7 @@ int Plan::choose_csr(const std::vector<int> &h_rp) {
       return panel_build(val_type, rows, m, n, nnz, a0, a1, val, exec, h_rp.data(), force, rule,
                          panel, &chosen, nullptr, lay);
     };
-    // x in FP64, layout and panel height left to the chooser: sorted groups
-    // where they are the better layout, whatever the x window's width.  A lane
-    // owns a row, so long runs of a row in a slice (narrow bands) cost it
-    // nothing, where the row-order body has one thread sum them.  They want
-    // every panel resident at once, a group of 64 rows for each of the four
-    // waves, and 4096 elements a panel.  us, row blocks / row order / sorted:
-    //   FP64 300,000 rows of 27, band 2,000:     25.0 /  23.2 /  21.3
-    //        300,000 of 140, band 3,800:        115.9 / 173.4 /  87.8
-    //        300,000 of 140, band 60,000:       194.8 / 117.4 / 110.3
-    //        512,000 of 27, band 13,000:         60.8 /  39.1 /  36.4
-    //        1,000,000 of 7, band 5,000:         29.0 /  26.9 /  22.8
-    //        1,000,000 of 140, band 5,000:      401.6 / 545.5 / 255.9
-    //   100,000 of 140 (two groups a panel), band 500: 32.7 / 84.2 / 40.6
-    //   500,000 of 4 (2048 elements a panel):          10.3 / 11.9 / 10.1
-    // In several rounds they lose to row order unless a row has more than 18
-    // elements in a slice.  2,000,000 rows, row order / sorted, by that number:
-    //   2.7: 500 / 600 (140 a row)   6.7: 116 / 125 (30)   10.5: 211 / 223 (60)
-    //   13.1: 394 / 424   17.9: 410 / 418   22.9: 550 / 415   28.2: 597 / 414 (120)
-    auto build_sorted64 = [&](double span) -> int {
-      if (opts.variant != 0 || opts.panel_rows > 0 || lo_opt != 0 || stats.max_row > kPanelCols)
-        return SBLAS_OK;
-      int rounds = 1;
-      const int rows = panel_rows_for(val_type, m, device, false, kPanelSorted, C, &rounds);
-      if (rows < 256) return SBLAS_OK;
-      return build(rows, PanelRule{min_panels, span, 4096, rounds > 1 ? 18.0 : 0.0}, kPanelSorted);
-    };
-    if (!narrow_x) st = build_sorted64(0.0);
+    if (!narrow_x) st = build_sorted64(h_rp, &chosen);
     if (st == SBLAS_OK && !chosen) {
       const int rows = opts.panel_rows > 0
                            ? opts.panel_rows
@@ -1070,12 +1132,10 @@ int Plan::choose_csr(const std::vector<int> &h_rp) {
            r2 *= 2)
         st = build(r2, rule, layout);
     }
-    if (st == SBLAS_OK && !chosen && narrow_x && narrow_x_asked() == 0) {
-      // narrow bands of narrow values: the forms tried below would mostly read
-      // x in FP64, and so do these panels (BF16, 1,000,000 rows of 140, band
-      // 5,000: 137 us against 296 for row blocks; 300,000 rows of 27, band
-      // 2,000: 15.3 against 18.7)
-      st = build_sorted64(0.0);
+    // narrow values on fewer elements than a trial takes: row blocks read x in
+    // FP64 there, and so do panels on narrow bands (more elements: band_panels)
+    if (st == SBLAS_OK && !chosen && narrow_x && narrow_x_asked() == 0 && nnz < (int64_t{1} << 20)) {
+      st = build_sorted64(h_rp, &chosen);
       narrow_x = false;
     }
     if (st == SBLAS_ERR_UNSUPPORTED && opts.variant == 0) {
@@ -1103,17 +1163,7 @@ int Plan::choose_csr(const std::vector<int> &h_rp) {
       panel.x32 = static_cast<float *>(p);
     }
     if (chosen) {
-      variant = 3;
-      int remap = opts.xcd_remap;
-      if (remap < 0) remap = env_int("SBLAS_XCD_REMAP", 1);
-      vl.xcd_remap = remap ? 1 : 0;
-      // rows cut by chunk edges: partials of their panels, merged in panel order
-      std::vector<int> mrows, mptr, mslots;
-      merge_lists(panel.hpanels, h_rp.data(), mrows, mptr, mslots);
-      pgroups = static_cast<int>(mrows.size());
-      if ((st = upload(*this, &d_pmrows, mrows)) != SBLAS_OK) return st;
-      if ((st = upload(*this, &d_pmptr, mptr)) != SBLAS_OK) return st;
-      if ((st = upload(*this, &d_pmslots, mslots)) != SBLAS_OK) return st;
+      if ((st = use_panels(h_rp)) != SBLAS_OK) return st;
       return setup_stream(h_rp.data());  // row blocks serve multi-RHS products
     }
   }
@@ -1155,6 +1205,11 @@ int Plan::choose_csr(const std::vector<int> &h_rp) {
     tuned = 3;
     rows_x32 = found.rows_x32;
     for (int i = 0; i < 4; i++) trial_ms[i] = found.ms[i];
+    if (val_type != SBLAS_VAL_F64 && narrow == 0 && !rows_x32) {
+      bool chosen = false;
+      if ((st = band_panels(h_rp, &chosen)) != SBLAS_OK) return st;
+      if (chosen) return use_panels(h_rp);
+    }
     if (found.kernel == SBLAS_KERNEL_CSR5) {
       kernel = SBLAS_KERNEL_CSR5;
       return setup_csr5(h_rp);
@@ -1211,22 +1266,13 @@ int Plan::choose_csr(const std::vector<int> &h_rp) {
   if ((st = trial(forms, ms)) != SBLAS_OK) return st;
   tuned = 2;
   for (size_t f = 0; f < forms.size(); f++) trial_ms[f] = ms[f];
-  // Narrow values: the forms over row blocks may gather x from an FP32 copy
+  // Narrow values: row blocks and segments may gather x from an FP32 copy
   // (normwise error 2.2e-8), the CSR5-style and column-sorted forms read x in
-  // FP64.  The copy is taken only where it clearly pays, so a matrix whose
-  // forms tie does not get one accuracy or the other by the noise of a trial:
-  // row blocks or segments a tenth ahead of the column-sorted form on x of
-  // 16 MB or more (R-MAT scale 22 0.6 of it, four a row in a band 0.83), row
-  // blocks 15 % ahead on smaller x with rows that are not very uneven (power
-  // law, 200,000 rows 0.75; banded, 100,000 rows of 140 0.87: FP64).  R-MAT
-  // matrices of smaller x (row CV about 9) keep FP64: the copy is worth 1 to
-  // 8 % there.
+  // FP64 (rows_take_x32).  Segments join the rule from 16 MB of x on.
   const bool auto_x = val_type != SBLAS_VAL_F64 && narrow == 0;
   if (auto_x) {
-    if (x_bytes >= (int64_t{16} << 20))
-      rows_x32 = std::min(ms[0], forms.size() > 3 ? ms[3] : ms[0]) < 0.9f * ms[2];
-    else
-      rows_x32 = stats.cv < 6.0 && ms[0] < 0.85f * ms[2];
+    const bool seg_too = forms.size() > 3 && x_bytes >= (int64_t{16} << 20);
+    rows_x32 = rows_take_x32(ms[0], seg_too ? ms[3] : 0.f, ms[2]);
   }
   const bool only_rows = auto_x && rows_x32;
   size_t best = 0;
@@ -1236,12 +1282,18 @@ int Plan::choose_csr(const std::vector<int> &h_rp) {
   }
   kernel = forms[best].first;
   variant = forms[best].second;
-  if (kernel != SBLAS_KERNEL_CSR5) drop_csr5(mark);
-  if (variant != 4) drop_sorted();
-  if (variant != 6 && !seg.buffers.empty()) drop_segments();
-  std::lock_guard<std::mutex> lk(g_tune_mu);
-  g_tune_cache[key] = TuneResult{kernel, variant, rows_x32, {trial_ms[0], trial_ms[1], trial_ms[2], trial_ms[3]}};
-  return SBLAS_OK;
+  {
+    std::lock_guard<std::mutex> lk(g_tune_mu);
+    g_tune_cache[key] = TuneResult{kernel, variant, rows_x32, {trial_ms[0], trial_ms[1], trial_ms[2], trial_ms[3]}};
+  }
+  bool panels = false;
+  if (auto_x && !rows_x32) {
+    if ((st = band_panels(h_rp, &panels)) != SBLAS_OK) return st;
+  }
+  if (kernel != SBLAS_KERNEL_CSR5 || panels) drop_csr5(mark);
+  if (variant != 4 || panels) drop_sorted();
+  if ((variant != 6 || panels) && !seg.buffers.empty()) drop_segments();
+  return panels ? use_panels(h_rp) : static_cast<int>(SBLAS_OK);
 }
 
 bool Plan::uses_tiles(int k) const {

@@ -166,6 +166,10 @@ struct Plan {
   int setup_tiles();
   int setup_csr5(const std::vector<int> &h_rp);
   int narrow_x_asked() const;
+  bool rows_take_x32(float rows_ms, float seg_ms, float sorted_ms) const;
+  int build_sorted64(const std::vector<int> &h_rp, bool *chosen);
+  int use_panels(const std::vector<int> &h_rp);
+  int band_panels(const std::vector<int> &h_rp, bool *chosen);
   int finish_csr(const std::vector<int> &h_rp);
   int choose_csr(const std::vector<int> &h_rp);
   void free_buffers_from(size_t first);
