@@ -130,6 +130,10 @@ int seg_build(int val_type, int m, int n, int64_t nnz, const int *rp, const int 
               const void *val, int P, SegmentFormat &f, std::vector<int> &h_vrp);
 // y[r] = alpha * (f.yv over r's virtual rows, segments ascending) + beta*y[r]
 int launch_seg_merge(const SegmentFormat &f, double alpha, double beta, double *y, hipStream_t s);
+// the same for k = 2 or 4 vectors: sums [f.M][k], Y [f.m][k]
+constexpr int kSegVectors = 4;
+int launch_seg_merge_vectors(const SegmentFormat &f, int k, const double *sums, double alpha,
+                             double beta, double *Y, hipStream_t s);
 // k in {2, 4, 8, 16} right-hand sides over the same row blocks; partials hold
 // 2 slots x k per block.
 int launch_csr_blocks_mrhs(int val_type, int k, const StreamLaunch &L, const RowBlock *blocks,

@@ -586,6 +586,20 @@ int Plan::run_spmm(int k, double alpha, const double *X, double beta, double *Y,
     }
     return SBLAS_OK;
   }
+  if (segment_vectors(k)) {
+    hipEvent_t *te = timing_slot();
+    if (te) SBLAS_HIP_TRY(hipEventRecord(te[0], s));
+    st = launch_csr_blocks_mrhs(val_type, k, vsl, d_vblocks, seg.vrp, seg.vcol, seg.vval, X,
+                                d_vsums, 1.0, 0.0, d_vkpartials, s);
+    if (st == SBLAS_OK && vgroups > 0)
+      st = launch_merge(d_vmrows, d_vmptr, d_vmslots, vgroups, d_vkpartials, k, d_vsums, 1.0, 0.0,
+                        s);
+    if (st == SBLAS_OK) st = launch_seg_merge_vectors(seg, k, d_vsums, alpha, beta, Y, s);
+    if (st != SBLAS_OK) return st;
+    if (te) SBLAS_HIP_TRY(hipEventRecord(te[1], s));
+    launches += 2 + (vgroups > 0 ? 1 : 0);
+    return SBLAS_OK;
+  }
   if (const int each = panel_vectors(k)) {
     hipEvent_t *te = timing_slot();
     if (te) SBLAS_HIP_TRY(hipEventRecord(te[0], s));
@@ -834,13 +848,50 @@ int Plan::setup_segments(int P) {
   return SBLAS_OK;
 }
 
+// Sums and partial slots of multi-vector products over the segments, for a plan
+// that has settled on them; without room for them those products keep the row
+// blocks.
+void Plan::setup_segment_vectors() {
+  void *p[2] = {nullptr, nullptr};
+  const size_t bytes[2] = {sizeof(double) * kSegVectors * static_cast<size_t>(seg.M),
+                           sizeof(double) * kSegVectors * 2 * static_cast<size_t>(vsl.nblocks)};
+  for (int i = 0; i < 2; i++)
+    if (hipMalloc(&p[i], std::max<size_t>(bytes[i], 8)) != hipSuccess) {
+      (void)hipGetLastError();
+      if (p[0] && i > 0) (void)hipFree(p[0]);
+      return;
+    }
+  for (int i = 0; i < 2; i++) {
+    seg.buffers.push_back(p[i]);
+    seg.bytes += static_cast<int64_t>(bytes[i]);
+    workspace_bytes += static_cast<int64_t>(bytes[i]);
+  }
+  d_vsums = static_cast<double *>(p[0]);
+  d_vkpartials = static_cast<double *>(p[1]);
+}
+
+// Multi-vector products over the segments: a virtual row costs k sums written and
+// read again, which two vectors always gain back, four where a row meets three
+// segments or more (columns spread evenly: most of their gathers miss L2
+// otherwise), and eight nowhere.  us, row blocks / segments at k = 2, 4, 8:
+//   power law 1,100,000 rows (3.1 pieces a row) 265 / 157  306 / 236  343 / 362
+//     1,900,000 (4.1) 510 / 290  562 / 454  606 / 682
+//     4,000,000 FP32 (5.6) 1169 / 728  1219 / 1081  1269 / 1598
+//   R-MAT 1,500,001 rows (1.7) 218 / 200  251 / 255  390 / 376
+//     3,000,000 (1.7) 253 / 250  370 / 406  527 / 576
+//     scale 22 (2.2) 687 / 631  917 / 884  1154 / 1153
+bool Plan::segment_vectors(int k) const {
+  if (variant != 6 || !d_vsums || !streams.empty()) return false;
+  return k == 2 || (k == 4 && seg.M >= 3 * static_cast<int64_t>(m));
+}
+
 void Plan::drop_segments() {
   for (void *p : seg.buffers) (void)hipFree(p);
   workspace_bytes -= seg.bytes;
   seg = SegmentFormat{};
   d_vblocks = nullptr;
   d_vmrows = d_vmptr = d_vmslots = nullptr;
-  d_vpartials = nullptr;
+  d_vpartials = d_vsums = d_vkpartials = nullptr;
   vgroups = 0;
   vsl = StreamLaunch{};
 }
@@ -1049,6 +1100,7 @@ int Plan::band_panels(const std::vector<int> &h_rp, bool *chosen) {
 int Plan::finish_csr(const std::vector<int> &h_rp) {
   int st = choose_csr(h_rp);
   if (st != SBLAS_OK) return st;
+  if (variant == 6 && seg.M > 0) setup_segment_vectors();
   // narrow values in row blocks: x gathered from an FP32 copy written by each
   // product unless asked not to (narrow_x 1; SBLAS_NARROW_X overrides the
   // auto setting).  R-MAT scale 22: FP32 values 1.10x -> 1.18x the FP64 plan,
@@ -1303,7 +1355,8 @@ bool Plan::uses_tiles(int k) const {
 
 bool Plan::has_merge(int k) const {
   if (uses_tiles(k)) return tiles > 0;
-  if (variant == 6 && k == 1 && streams.empty()) return false;  // merges run inside the product
+  if ((variant == 6 && k == 1 && streams.empty()) || segment_vectors(k))
+    return false;  // merges run inside the product
   if ((variant == 3 && k == 1 && streams.empty()) || panel_vectors(k)) return pgroups > 0;
   if (variant == 4 && k == 1 && streams.empty()) return sgroups > 0;
   if (variant >= 2 && streams.empty())  // row blocks (any k)
@@ -1312,7 +1365,7 @@ bool Plan::has_merge(int k) const {
 }
 
 int Plan::run_merge(int k, double alpha, double beta, double *Y, hipStream_t s) {
-  if (variant == 6 && k == 1 && streams.empty()) return SBLAS_OK;
+  if ((variant == 6 && k == 1 && streams.empty()) || segment_vectors(k)) return SBLAS_OK;
   if (uses_tiles(k))
     return tiles > 0 ? launch_tile_fixup(carry_count(), d_carry, Y, alpha, beta, s) : SBLAS_OK;
   if ((variant == 3 && k == 1 && streams.empty()) || panel_vectors(k))

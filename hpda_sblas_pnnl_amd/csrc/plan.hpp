@@ -107,6 +107,8 @@ struct Plan {
   int *d_vmrows = nullptr, *d_vmptr = nullptr, *d_vmslots = nullptr;
   int vgroups = 0;
   double *d_vpartials = nullptr;
+  double *d_vsums = nullptr;          // [seg.M][kSegVectors] of a multi-vector product, or nullptr
+  double *d_vkpartials = nullptr;     // its partial slots
 
   // CSR5-style format (kernel 3)
   uint32_t *d_c5_tile_nz = nullptr, *d_c5_flags = nullptr;
@@ -178,6 +180,8 @@ struct Plan {
   void drop_csr5(size_t mark);
   int setup_segments(int P);
   void drop_segments();
+  void setup_segment_vectors();
+  bool segment_vectors(int k) const;
   // times the given (kernel, variant) forms on the plan's own matrix; ms[i]
   // receives the median of form i
   int trial(const std::vector<std::pair<int, int>> &forms, std::vector<float> &ms);
