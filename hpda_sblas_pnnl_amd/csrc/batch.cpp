@@ -308,8 +308,19 @@ int sblas_batch_create(int count, const sblas_batch_item *items, const sblas_opt
     if (narrow && !(opts && opts->panel_rows > 0) &&
         (static_cast<int64_t>(it.m) + solo_rows - 1) / solo_rows < cus)
       narrow = false;
+    // Row-order panels only for rows of even length (CV at most 1) unless asked
+    // for: one thread sums a row's run in a slice while its workgroup waits, and a
+    // batch's few panels have nothing beside them.  us a batch, panels / row
+    // blocks, FP64: eight R-MAT matrices of 13,594 rows 662 / 18, power law 14,000
+    // rows 290 / 18, 30,000 194 / 28, 80,000 216 / 61; log-normal rows of 60, CV 1.5
+    // 316 / 78; four of 200,000 rows of 100, CV 1.5 582 / 387, CV 0.8 422 / 390.
+    // Narrow values build the panels all the same: where they would have been
+    // taken, the row blocks read x in FP64 as they do.
+    const bool asked = want == 3 || (opts && opts->panel_rows > 0);
+    const bool row_order = asked || rs.cv <= 1.0;
+    bool x64 = false;
     if (kv == 1 && it.m > 0 && it.nnz > 0 && want != 1 && want != 2 &&
-        (want == 3 || rs.max_row <= 8192)) {
+        (want == 3 || rs.max_row <= 8192) && (row_order || it.val_type != SBLAS_VAL_F64)) {
       const std::vector<ExecChunk> one{ExecChunk{0, it.nnz, 0, it.m}};
       int rows = (opts && opts->panel_rows > 0) ? std::min(opts->panel_rows, kBatchPanelRowsMax)
                  : narrow ? solo_rows
@@ -348,6 +359,10 @@ int sblas_batch_create(int count, const sblas_batch_item *items, const sblas_opt
       }
       if (st == SBLAS_OK && panel && layout == kPanelRowOrder && !f.srp)
         panel = false;  // slices beyond 16-bit offsets
+      if (st == SBLAS_OK && panel && layout == kPanelRowOrder && !row_order) {
+        panel = false;
+        x64 = true;
+      }
       if (st == SBLAS_ERR_UNSUPPORTED && want != 3) {
         clear_error();
         st = SBLAS_OK;
@@ -407,8 +422,8 @@ int sblas_batch_create(int count, const sblas_batch_item *items, const sblas_opt
     } else {
       // narrow values in row blocks gather x from an FP32 copy (as a plan
       // does for matrices of 2^20 elements or more)
-      if (it.val_type != SBLAS_VAL_F64 && nxo == 2 && kv == 1 && it.nnz >= (int64_t{1} << 20) &&
-          it.n > 0) {
+      if (it.val_type != SBLAS_VAL_F64 && nxo == 2 && !x64 && kv == 1 &&
+          it.nnz >= (int64_t{1} << 20) && it.n > 0) {
         void *p = nullptr;
         if (hipMalloc(&p, sizeof(float) * static_cast<size_t>(it.n)) != hipSuccess) {
           set_error(SBLAS_ERR_ALLOC, "batch: FP32 x copy allocation failed");
