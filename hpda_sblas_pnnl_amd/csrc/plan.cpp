@@ -998,14 +998,16 @@ int Plan::narrow_x_asked() const {
 // where row blocks that sum rows by lane groups beat the column-sorted form; a
 // faster row-block kernel must not take FP64 x from the matrices that had it,
 // so those times are put back: rows * (0.975 + 0.104 where x fits in an XCD's
-// L2, less beyond) + 1.8 us for each unit of the rows' CV above 4 + 0.25 us,
-// within 9 % on 28 of 29 matrices (banded, power law, R-MAT; 1 to 43 M elements,
-// rows 8 to 240 us).  By these estimates the matrices that had the copy lie
-// below 0.94 of the column-sorted form, those with x in FP64 above 0.99, but for
-// two R-MAT ties (1.01 and 1.00) that now read x in FP64.
+// L2, less beyond, + 0.06 for rows of a CV from 0.12 to 4, whose lane groups
+// waited) + 1.8 us for each unit of the CV above 4 + 0.25 us.  On 48 matrices
+// (banded, power law, R-MAT; 1 to 43 M elements, rows 8 to 240 us) those that had
+// x in FP64 lie at 0.99 of the column-sorted form or above, those that had the
+// copy below 0.96 but for five close ones (0.98 to 1.02), which read x in FP64
+// now.
 bool Plan::rows_take_x32(float rows_ms, float seg_ms, float sorted_ms) const {
   const double share = std::min(1.0, static_cast<double>(4 << 20) / (8.0 * std::max(n, 1)));
-  double t = rows_ms * (0.975 + 0.104 * share) + 1.8e-3 * std::max(0.0, stats.cv - 4.0) + 2.5e-4;
+  const double waits = stats.cv >= 0.12 && stats.cv <= 4.0 ? 0.06 : 0.0;
+  double t = rows_ms * (0.975 + 0.104 * share + waits) + 1.8e-3 * std::max(0.0, stats.cv - 4.0) + 2.5e-4;
   if (seg_ms > 0.f) t = std::min(t, 1.03 * static_cast<double>(seg_ms));
   return t < 0.96 * static_cast<double>(sorted_ms);
 }
