@@ -24,6 +24,7 @@ ARCH = os.environ.get("SBLAS_OFFLOAD_ARCH", "gfx950")
 
 HIP_SOURCES = [
     "sblas_vector.hip",
+    "sblas_lanes.hip",
     "sblas_spmm.hip",
     "sblas_tiles.hip",
     "sblas_csc.hip",

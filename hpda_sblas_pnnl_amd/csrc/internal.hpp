@@ -65,7 +65,7 @@ constexpr int kStreamRowsMax = 1024;   // rows per row block (LDS y staging)
 
 struct StreamLaunch {
   int items;        // elements per thread: block holds 256*items elements
-  int subwave;      // lanes per row in the LDS reduction (1..64)
+  int subwave;      // lanes per row of launch_csr_lanes (1..64)
   int nblocks;
   int grid;
   int xcd_remap;
@@ -100,6 +100,12 @@ int launch_csr_stream(int val_type, const StreamLaunch &L, const RowBlock *block
                       const int *rp, const int *col, const void *val, const double *x,
                       double *y, double alpha, double beta, double *partials, hipStream_t s,
                       const float *x32 = nullptr);
+// The same product with rows summed by groups of L.subwave lanes and x in FP64
+// (FP32 / BF16 values): timed by a plan's trial, run by no product
+// (sblas_lanes.hip).
+int launch_csr_lanes(int val_type, const StreamLaunch &L, const RowBlock *blocks, const int *rp,
+                     const int *col, const void *val, const double *x, double *y, double alpha,
+                     double beta, double *partials, hipStream_t s);
 // x32[i] = x[i] rounded to FP32, i < n
 int launch_x_to_f32(int n, const double *x, float *x32, hipStream_t s);
 // Row blocks over column segments (sblas_segment.hip): the elements of row r

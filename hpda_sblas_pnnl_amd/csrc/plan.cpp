@@ -950,6 +950,7 @@ int Plan::trial(const std::vector<std::pair<int, int>> &forms, std::vector<float
   const bool was_timing = timing;
   timing = false;
   auto run_as = [&](const std::pair<int, int> &f) {
+    if (f.second < 0) return run_lanes(f.second == kLaneSegments, tx, ty, ts);
     kernel = f.first;
     variant = f.second;
     return run_spmm(1, 1.0, tx, 0.0, ty, ts);
@@ -993,23 +994,21 @@ int Plan::narrow_x_asked() const {
   return opts.narrow_x != 0 ? opts.narrow_x : std::max(env_int("SBLAS_NARROW_X", 0), 0);
 }
 
-// Whether narrow values in row blocks (or segments; 0: not among the forms)
-// gather x from an FP32 copy, by the trial's times in ms.  A matrix had the copy
-// where row blocks that sum rows by lane groups beat the column-sorted form; a
-// faster row-block kernel must not take FP64 x from the matrices that had it,
-// so those times are put back: rows * (0.975 + 0.104 where x fits in an XCD's
-// L2, less beyond, + 0.06 for rows of a CV from 0.12 to 4, whose lane groups
-// waited) + 1.8 us for each unit of the CV above 4 + 0.25 us.  On 48 matrices
-// (banded, power law, R-MAT; 1 to 43 M elements, rows 8 to 240 us) those that had
-// x in FP64 lie at 0.99 of the column-sorted form or above, those that had the
-// copy below 0.96 but for five close ones (0.98 to 1.02), which read x in FP64
-// now.
-bool Plan::rows_take_x32(float rows_ms, float seg_ms, float sorted_ms) const {
-  const double share = std::min(1.0, static_cast<double>(4 << 20) / (8.0 * std::max(n, 1)));
-  const double waits = stats.cv >= 0.12 && stats.cv <= 4.0 ? 0.06 : 0.0;
-  double t = rows_ms * (0.975 + 0.104 * share + waits) + 1.8e-3 * std::max(0.0, stats.cv - 4.0) + 2.5e-4;
-  if (seg_ms > 0.f) t = std::min(t, 1.03 * static_cast<double>(seg_ms));
-  return t < 0.96 * static_cast<double>(sorted_ms);
+// y = A*x over the row blocks, or over the segments, with rows summed by groups
+// of lanes (sblas_lanes.hip): what the trial times for the x precision of narrow
+// values.
+int Plan::run_lanes(bool segments, const double *x, double *y, hipStream_t s) {
+  if (!segments) {
+    int st = launch_csr_lanes(val_type, sl, d_rblocks, a0, a1, val, x, y, 1.0, 0.0, d_bpartials, s);
+    if (st == SBLAS_OK && bgroups > 0)
+      st = launch_merge(d_bmrows, d_bmptr, d_bmslots, bgroups, d_bpartials, 1, y, 1.0, 0.0, s);
+    return st;
+  }
+  int st = launch_csr_lanes(val_type, vsl, d_vblocks, seg.vrp, seg.vcol, seg.vval, x, seg.yv, 1.0,
+                            0.0, d_vpartials, s);
+  if (st == SBLAS_OK && vgroups > 0)
+    st = launch_merge(d_vmrows, d_vmptr, d_vmslots, vgroups, d_vpartials, 1, seg.yv, 1.0, 0.0, s);
+  return st == SBLAS_OK ? launch_seg_merge(seg, 1.0, 0.0, y, s) : st;
 }
 
 // x in FP64, layout and panel height left to the chooser: sorted groups
@@ -1316,21 +1315,38 @@ int Plan::choose_csr(const std::vector<int> &h_rp) {
       forms.push_back({SBLAS_KERNEL_VECTOR, 6});
     }
   }
-  std::vector<float> ms;
-  if ((st = trial(forms, ms)) != SBLAS_OK) return st;
-  tuned = 2;
-  for (size_t f = 0; f < forms.size(); f++) trial_ms[f] = ms[f];
   // Narrow values: row blocks and segments may gather x from an FP32 copy
   // (normwise error 2.2e-8), the CSR5-style and column-sorted forms read x in
-  // FP64 (rows_take_x32).  Segments join the rule from 16 MB of x on.
+  // FP64.  Which of the two a matrix gets must not follow the speed of the kernels
+  // that multiply, so it has a measure of its own: the copy where rows summed by
+  // groups of lanes (over segments too from 16 MB of x) are not slower than the
+  // column-sorted form.  They are timed first: the launch after an idle GPU takes
+  // up to 1 us more, as it did when only the trial's forms were timed; the launch
+  // between takes about 0.5 % off the column-sorted form, put back here.  Ties
+  // fall to either side from process to process (of 134 narrow matrices, ten lie
+  // within 1.5 %, one of them R-MAT, 1,500,001 rows, BF16: 171.1 / 170.7, 170.7 /
+  // 171.9, 171.0 / 172.1 us in three trials).
   const bool auto_x = val_type != SBLAS_VAL_F64 && narrow == 0;
+  const size_t count = forms.size();
+  std::vector<std::pair<int, int>> timed = forms;
   if (auto_x) {
-    const bool seg_too = forms.size() > 3 && x_bytes >= (int64_t{16} << 20);
-    rows_x32 = rows_take_x32(ms[0], seg_too ? ms[3] : 0.f, ms[2]);
+    timed.insert(timed.begin(), {SBLAS_KERNEL_VECTOR, kLaneRows});
+    if (count > 3 && x_bytes >= (int64_t{16} << 20))
+      timed.push_back({SBLAS_KERNEL_VECTOR, kLaneSegments});
   }
+  std::vector<float> ms;
+  if ((st = trial(timed, ms)) != SBLAS_OK) return st;
+  tuned = 2;
+  if (auto_x) {
+    float lanes = ms[0];
+    if (timed.size() > count + 1) lanes = std::min(lanes, ms[count + 1]);
+    ms.erase(ms.begin());
+    rows_x32 = lanes <= 1.005f * ms[2];
+  }
+  for (size_t f = 0; f < count; f++) trial_ms[f] = ms[f];
   const bool only_rows = auto_x && rows_x32;
   size_t best = 0;
-  for (size_t f = 1; f < forms.size(); f++) {
+  for (size_t f = 1; f < count; f++) {
     const bool rows = f == 3;
     if (ms[f] < ms[best] && (rows || !only_rows)) best = f;
   }

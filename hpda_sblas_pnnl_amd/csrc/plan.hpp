@@ -168,7 +168,7 @@ struct Plan {
   int setup_tiles();
   int setup_csr5(const std::vector<int> &h_rp);
   int narrow_x_asked() const;
-  bool rows_take_x32(float rows_ms, float seg_ms, float sorted_ms) const;
+  int run_lanes(bool segments, const double *x, double *y, hipStream_t s);
   int build_sorted64(const std::vector<int> &h_rp, bool *chosen);
   int use_panels(const std::vector<int> &h_rp);
   int band_panels(const std::vector<int> &h_rp, bool *chosen);
@@ -183,7 +183,9 @@ struct Plan {
   void setup_segment_vectors();
   bool segment_vectors(int k) const;
   // times the given (kernel, variant) forms on the plan's own matrix; ms[i]
-  // receives the median of form i
+  // receives the median of form i.  Variants kLaneRows and kLaneSegments stand
+  // for run_lanes.
+  static constexpr int kLaneRows = -2, kLaneSegments = -6;
   int trial(const std::vector<std::pair<int, int>> &forms, std::vector<float> &ms);
   int run_merge(int k, double alpha, double beta, double *Y, hipStream_t s);
   hipEvent_t *timing_slot();
