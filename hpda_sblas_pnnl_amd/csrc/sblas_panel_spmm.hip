@@ -77,8 +77,11 @@ __global__ __launch_bounds__(spmm_threads<K>()) void k_panel_spmm(
   const int t = threadIdx.x, w = t >> 6, l = t & 63, wv = t & ~63;
   const bool x16 = (reinterpret_cast<uintptr_t>(X) & 15) == 0;  // a row is an even number of doubles
   const int s0 = slice_base[p], s1 = slice_base[p + 1];
-  // the sums, and the row of X that padding meets
+  // the sums, and the row of X that padding meets; the barrier outside the
+  // slices, since a panel of empty rows has none and its sums are read below all
+  // the same
   for (int i = t; i < (R + 1) * K; i += T) xs[W * K + i] = 0.0;
+  __syncthreads();
 
   for (int s = s0; s < s1; s++) {
     const int64_t sb = slice_off[s];
