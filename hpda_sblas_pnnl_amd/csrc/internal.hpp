@@ -267,6 +267,8 @@ struct PanelFormat {
   std::vector<void *> buffers;
 };
 int panel_rpt(int rows);
+// Time in us that an element of a row adds to its lane in the sorted layout.
+double panel_chain_us(int rows);
 // Rows per row panel so the panels fill whole rounds of resident workgroups;
 // *rounds (sorted layout, may be null) = how many.
 int panel_rows_for(int val_type, int m, int device, bool narrow_x = false,
@@ -276,17 +278,23 @@ int panel_rows_for(int val_type, int m, int device, bool narrow_x = false,
 int columns_ascend(int m, int64_t nnz, const int *rp, const int *col, hipStream_t s, bool *ok);
 // When the form pays: at least `panels` row panels, each of which on average
 // spans more than `span` column panels, holds `elements` elements and, per row
-// and slice, `per_row` elements (beside the rules of panel_build itself).
+// and slice, `per_row` elements, and none more than `dense` times the mean (or
+// `few` elements); `chain`: the longest row's chain of loads over the time that all
+// elements take to stream (beside the rules of panel_build itself).
 struct PanelRule {
   int panels = 1;
   double span = 3.0;
   int64_t elements = 0;
   double per_row = 0.0;
+  double dense = 4.0;
+  int64_t few = 65536;
+  double chain = 0.0;
 };
 // Builds the format on the device: each execution chunk of `ex` cut into row
 // panels of at most `rows` rows (h_rp: host copy of the row pointers).  With
 // force == false it stops after the per-panel column ranges and sets
-// *chosen = false when the form would not help (the rule, or sparse slices).
+// *chosen = false when the form would not help (the rule, sparse slices, or row
+// panels of very uneven density).
 // Also with force, *chosen = false for rows whose columns do not ascend: their
 // elements in a column panel would not be one run.
 // layout kPanelSorted rounds the rows per panel up to a multiple of 64.

@@ -1029,6 +1029,22 @@ int Plan::run_lanes(bool segments, const double *x, double *y, hipStream_t s) {
 // elements in a slice.  2,000,000 rows, row order / sorted, by that number:
 //   2.7: 500 / 600 (140 a row)   6.7: 116 / 125 (30)   10.5: 211 / 223 (60)
 //   13.1: 394 / 424   17.9: 410 / 418   22.9: 550 / 415   28.2: 597 / 414 (120)
+// A row's elements in a slice are one lane's chain of loads, 0.62 us a round and
+// 0.047 us an element, while the other panels have long finished.  The form wants
+// the longest row's chain below the time that all elements take to stream (6.05e11
+// of 10 bytes a second): at most 0.9 of it against row blocks, 0.6 where row order
+// would take the matrix.  The best other form / sorted, us, by that share:
+//   band 6,000 (row blocks, column-sorted)
+//     300,000 rows of 50     0.25 47 / 30   0.83 49 / 42   1.0 49 / 47   1.8 49 / 63
+//     600,000 of 60          0.20 99 / 64   0.84 106 / 89   1.4 106 / 123
+//     1,000,000 of 27        0.15 84 / 52   0.63 85 / 63   1.1 86 / 83   23 85 / 1018
+//   band 50,000 (row order)
+//     300,000 of 120         0.25 100 / 89   0.57 102 / 100   0.92 104 / 113
+//     1,000,000 of 60        0.15 142 / 124   0.60 147 / 147   1.0 143 / 189
+// And, all panels running at once, no panel may hold much more than its share (a
+// tenth of the rows 2 / 3 / 3.9 times as long as the mean, row blocks / sorted:
+// 512,000 rows of 27 47 / 42, 48 / 54, 48 / 67; 2,000,000 of 100 620 / 502, 625 /
+// 661, 616 / 805).
 int Plan::build_sorted64(const std::vector<int> &h_rp, bool *chosen) {
   *chosen = false;
   if (opts.variant != 0 || opts.panel_rows > 0 || opts.panel_layout != 0 ||
@@ -1039,10 +1055,13 @@ int Plan::build_sorted64(const std::vector<int> &h_rp, bool *chosen) {
   const int rows = panel_rows_for(val_type, m, device, false, kPanelSorted,
                                   static_cast<int>(exec.size()), &rounds);
   if (rows < 256) return SBLAS_OK;
+  PanelRule rule{2 * std::max(cus, 1), 0.0, 4096, rounds > 1 ? 18.0 : 0.0};
+  rule.dense = 2.25;
+  rule.few = 0;
+  rule.chain = stats.max_row * panel_chain_us(rows) / (std::max<int64_t>(nnz, 1) / 6.05e5);
   panel = PanelFormat{};
   return panel_build(val_type, rows, m, n, nnz, a0, a1, val, exec, h_rp.data(), false,
-                     PanelRule{2 * std::max(cus, 1), 0.0, 4096, rounds > 1 ? 18.0 : 0.0}, panel,
-                     chosen, nullptr, kPanelSorted);
+                     rule, panel, chosen, nullptr, kPanelSorted);
 }
 
 // The plan's products run over its column panels from now on.

@@ -483,12 +483,15 @@ int panel_build(int val_type, int rows, int m, int n, int64_t nnz, const int *rp
   // densest panel may hold at most 4x the mean, or 65536 elements.
   int64_t densest = 0;
   for (const int2 &w : hwin) densest = std::max<int64_t>(densest, w.y - w.x);
-  const bool balanced =
-      densest <= std::max<int64_t>(65536, 4 * nnz / std::max(f.npanels, 1));
+  const int64_t mean = nnz / std::max(f.npanels, 1);
+  const bool balanced = densest <= std::max(rule.few, static_cast<int64_t>(rule.dense * mean));
+  // a long chain weighs less against row blocks than against row order, which
+  // takes wide windows
+  const bool short_chain = rule.chain <= (f.avg_panels_per_row_panel > 3.0 ? 0.6 : 0.9);
   const bool helps = f.npanels >= rule.panels && f.avg_slice >= 1024.0 &&
                      f.avg_panels_per_row_panel > rule.span &&
                      nnz >= rule.elements * f.npanels && f.avg_slice >= rule.per_row * R &&
-                     balanced;
+                     balanced && short_chain;
   bool ascend = true;
   if (force || helps) {
     const int st = columns_ascend(m, nnz, rp, col, s, &ascend);
@@ -802,6 +805,7 @@ int panel_rpt(int rows) {
   const int need = (rows + 255) / 256;
   return need <= 1 ? 1 : need <= 2 ? 2 : need <= 4 ? 4 : need <= 6 ? 6 : 8;
 }
+double panel_chain_us(int rows) { return 0.047 + 0.62 / sorted_panel::unroll_for(panel_rpt(rows)); }
 
 namespace {
 // resident workgroups per CU of the sorted-group kernel with RPT rows per thread
