@@ -53,15 +53,18 @@ struct CallContext {
   char *dev = nullptr;
   size_t dev_bytes = 0;
 
-  bool ready(size_t bytes) {
+  bool ready(size_t bytes, size_t pinned_bytes = kPinnedBytes) {
     if (failed) return false;
     if (!stream) {
       failed = hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) != hipSuccess;
       for (hipEvent_t &e : ev) failed = failed || hipEventCreate(&e) != hipSuccess;
       void *p = nullptr;
-      failed = failed || hipHostMalloc(&p, kPinnedBytes, hipHostMallocDefault) != hipSuccess;
+      failed = failed || hipHostMalloc(&p, pinned_bytes, hipHostMallocDefault) != hipSuccess;
       pinned = static_cast<char *>(p);
-      if (failed) return false;
+    }
+    if (failed) {
+      (void)hipGetLastError();  // the plan path's launches must not find it
+      return false;
     }
     if (bytes > dev_bytes) {
       if (dev) (void)hipFree(dev);
@@ -70,7 +73,7 @@ struct CallContext {
       const size_t want = (bytes + (size_t{1} << 20) - 1) >> 20 << 20;
       void *p = nullptr;
       if (hipMalloc(&p, want) != hipSuccess) {
-        (void)hipGetLastError();  // the plan path's launches must not find it
+        (void)hipGetLastError();
         return false;
       }
       dev = static_cast<char *>(p);
@@ -355,3 +358,16 @@ int direct_csr(int device, int m, int n, int nnz, double alpha, const double *va
 }
 
 }  // namespace sblas
+
+// The HIP error that a call context leaves behind whose pinned buffer cannot be had,
+// -1 if it can (not in sblas.h; used by the tests).
+extern "C" int sblas_internal_call_context_error(size_t pinned_bytes) {
+  sblas::CallContext c;
+  const bool ok = c.ready(0, pinned_bytes);
+  const int left = static_cast<int>(hipGetLastError());
+  for (hipEvent_t e : c.ev)
+    if (e) (void)hipEventDestroy(e);
+  if (c.stream) (void)hipStreamDestroy(c.stream);
+  if (ok) (void)hipHostFree(c.pinned);
+  return ok ? -1 : left;
+}
