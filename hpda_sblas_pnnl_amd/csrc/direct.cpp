@@ -40,7 +40,7 @@ constexpr size_t kContextBytes = size_t{64} << 20;  // device memory of a contex
 constexpr size_t kPinnedBytes = size_t{1} << 20;    // its pinned buffer
 constexpr size_t kFlagAt = kPinnedBytes - 64;       // the index flag's place there
 constexpr int kMaxDevices = 64;
-constexpr int kEvents = 8;
+constexpr int kEvents = 7;
 
 // Contexts live until the process ends: no HIP call runs from a static
 // destructor.
@@ -135,7 +135,6 @@ int failed(const char *what) {
 int run(CallContext &c, int m, int n, int nnz, double alpha, const double *val,
         const int *rp, const int *col, const double *x, double beta, double *y, int kernel,
         int part_mode, spmv_ret &ret, bool &handled) {
-  const double t0 = now_s();
   const bool merge_path = kernel == SBLAS_KERNEL_MERGE, csr5 = kernel == SBLAS_KERNEL_CSR5;
   const char *ec = std::getenv("SBLAS_CHUNKS");
   const int C = std::max(1, ec && *ec ? std::atoi(ec) : 1);
@@ -165,6 +164,10 @@ int run(CallContext &c, int m, int n, int nnz, double alpha, const double *val,
     clear_error();
     return SBLAS_OK;
   }
+  // spmv_ret: comm_time the copies of the caller's arrays and y; part_time what a
+  // plan's creation would do, on the host (host_s, while the arrays are copied) and
+  // on the device (its lists uploaded, indices checked, a format laid out)
+  double host_s = -now_s();
   for (int r = 0; r < m; r++)
     if (rp[r + 1] < rp[r]) {
       handled = true;
@@ -178,7 +181,8 @@ int run(CallContext &c, int m, int n, int nnz, double alpha, const double *val,
   int *d_flag = reinterpret_cast<int *>(d + o_flag);
   double *d_val = reinterpret_cast<double *>(d + o_val);
   double *d_x = reinterpret_cast<double *>(d + o_x), *d_y = reinterpret_cast<double *>(d + o_y);
-  enum { UP_A, UP_B, COMP_A, COMP_B, MERGE_A, MERGE_B, DOWN_A, DOWN_B };
+  // an event costs about 6 us of a call, so neighbouring steps share theirs
+  enum { UP_A, UP_B, PREP_A, COMP_A, COMP_B, MERGE_B, DOWN_B };
   // whatever happens below, nothing of this call is left on the stream when
   // the context is handed on
   struct Drain {
@@ -186,6 +190,7 @@ int run(CallContext &c, int m, int n, int nnz, double alpha, const double *val,
     ~Drain() { (void)hipStreamSynchronize(s); }
   } drain{s};
 
+  host_s += now_s();
   (void)hipEventRecord(c.ev[UP_A], s);
   {
     StagingLease ring((sizeof(int) + sizeof(double)) * static_cast<size_t>(nnz) +
@@ -199,7 +204,9 @@ int run(CallContext &c, int m, int n, int nnz, double alpha, const double *val,
       return st;
     if (beta != 0.0 && (st = ring.to_device(d_y, y, sizeof(double) * m, s)) != SBLAS_OK) return st;
   }
+  (void)hipEventRecord(c.ev[UP_B], s);
   // what the kernel needs beside the matrix, while the transfers run
+  host_s -= now_s();
   int *flag_home = reinterpret_cast<int *>(c.pinned + kFlagAt);
   *flag_home = 0;
   StreamLaunch L{};
@@ -256,16 +263,19 @@ int run(CallContext &c, int m, int n, int nnz, double alpha, const double *val,
     }
     for (const Pack::Part &q : pack.parts)
       if (q.bytes) std::memcpy(stage + (q.at - pack.start), q.src, q.bytes);
+    host_s += now_s();
+    (void)hipEventRecord(c.ev[PREP_A], s);
     if (hipMemcpyAsync(d + pack.start, stage, pack_bytes, hipMemcpyHostToDevice, s) != hipSuccess ||
         (!large.empty() && hipStreamSynchronize(s) != hipSuccess))
       return failed("upload failed");
+  } else {
+    host_s += now_s();
+    (void)hipEventRecord(c.ev[PREP_A], s);
   }
   if (hipMemcpyAsync(d_flag, flag_home, sizeof(int), hipMemcpyHostToDevice, s) != hipSuccess)
     return failed("upload failed");
-  (void)hipEventRecord(c.ev[UP_B], s);
   int st = launch_sanitize_cols(nnz, d_col, n, d_flag, s);
   if (st != SBLAS_OK) return st;
-  ret.part_time = now_s() - t0;
 
   TileCarry *carry = reinterpret_cast<TileCarry *>(d + o_carry);
   double *partials = reinterpret_cast<double *>(d + o_part);
@@ -293,7 +303,6 @@ int run(CallContext &c, int m, int n, int nnz, double alpha, const double *val,
   (void)hipEventRecord(c.ev[COMP_B], s);
   const bool merged = merge_path || csr5 || groups > 0;
   if (merged) {
-    (void)hipEventRecord(c.ev[MERGE_A], s);
     st = merge_path ? launch_tile_fixup(tiles, carry, d_y, alpha, beta, s)
          : csr5     ? launch_csr5_finish((tiles + 3) / 4, carry, static_cast<int>(c5.empty.size()),
                                          ints(o_empty), alpha, beta, d_y, s)
@@ -306,7 +315,6 @@ int run(CallContext &c, int m, int n, int nnz, double alpha, const double *val,
   // flag and y, and y stays untouched when an index was out of range
   const size_t y_bytes = sizeof(double) * static_cast<size_t>(m);
   const bool by_pinned = y_bytes <= kFlagAt;
-  (void)hipEventRecord(c.ev[DOWN_A], s);
   if (hipMemcpyAsync(flag_home, d_flag, sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess ||
       (by_pinned &&
        hipMemcpyAsync(c.pinned, d_y, y_bytes, hipMemcpyDeviceToHost, s) != hipSuccess))
@@ -327,10 +335,11 @@ int run(CallContext &c, int m, int n, int nnz, double alpha, const double *val,
       return failed("download failed");
     y_s = now_s() - t1;
   }
-  ret.comm_time = seconds(c.ev[UP_A], c.ev[UP_B]) + seconds(c.ev[DOWN_A], c.ev[DOWN_B]) + y_s;
+  const int done = merged ? MERGE_B : COMP_B;
+  ret.part_time = host_s + seconds(c.ev[PREP_A], c.ev[COMP_A]);
+  ret.comm_time = seconds(c.ev[UP_A], c.ev[UP_B]) + seconds(c.ev[done], c.ev[DOWN_B]) + y_s;
   ret.comp_time = seconds(c.ev[COMP_A], c.ev[COMP_B]);
-  ret.merg_time = merged ? seconds(c.ev[MERGE_A], c.ev[MERGE_B]) : 0.0;
-  ret.part_time = std::max(0.0, ret.part_time - seconds(c.ev[UP_A], c.ev[UP_B]));
+  ret.merg_time = merged ? seconds(c.ev[COMP_B], c.ev[MERGE_B]) : 0.0;
   return SBLAS_OK;
 }
 

@@ -3,11 +3,12 @@
 //
 // Each call is synchronous and stateless like the reference's: the caller's
 // host arrays are uploaded, a plan is built (CSR matrices that with their
-// vectors take up to 64 MB go without one, direct.cpp) with the entry point's partition
-// rule at the configured chunk count (ngpu must be 1; chunks come from
+// vectors take up to 64 MB go without one, direct.cpp) with the entry point's
+// partition rule at the configured chunk count (ngpu must be 1; chunks come from
 // SBLAS_CHUNKS, default 1), the kernel runs on a private stream, split rows
 // are merged on the device and y is copied back.  spmv_ret holds the times of
-// those steps in seconds: part_time (partition + plan), comm_time (uploads and
+// those steps in seconds: part_time (partition + plan, or the same work without a
+// plan, whose host part runs beside the uploads), comm_time (uploads and
 // download), comp_time (kernels), merg_time (device merge of split rows).
 //
 // Semantics follow y = alpha*A*x + beta*y for every row, including the rows
@@ -91,7 +92,10 @@ spmv_ret run_format(int format, int m, int n, int nnz, const double *alpha, cons
     const int st = direct_csr(env_int("SBLAS_DEVICE", 0), m, n, nnz, *alpha, val, a0, a1, x,
                               *beta, y, kernel, part_mode, ret, handled);
     if (st != SBLAS_OK) return nan_ret();
-    if (handled) return ret;
+    if (handled) {
+      ret.part_time += host_prep_s;
+      return ret;
+    }
   }
   hipStream_t s = nullptr;
   if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) {
