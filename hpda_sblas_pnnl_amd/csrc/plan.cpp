@@ -130,6 +130,7 @@ Plan::~Plan() {
   for (void *p : sorted.buffers) (void)hipFree(p);
   for (void *p : seg.buffers) (void)hipFree(p);
   for (hipEvent_t e : tev) (void)hipEventDestroy(e);
+  if (last_event) (void)hipEventDestroy(last_event);
   for (void *p : device_buffers) (void)hipFree(p);
   for (hipStream_t s : streams) (void)hipStreamDestroy(s);
   for (hipEvent_t e : events) (void)hipEventDestroy(e);
@@ -492,6 +493,11 @@ int Plan::run_spmm(int k, double alpha, const double *X, double beta, double *Y,
   }
   int st = SBLAS_OK;
   const int C = static_cast<int>(exec.size());
+  std::unique_lock<std::mutex> order(order_mu, std::defer_lock);
+  if (shares_workspace(k)) {
+    order.lock();
+    if ((st = follow_last(s)) != SBLAS_OK) return st;
+  }
   if (uses_tiles(k)) {
     // COO segmented reduction or merge-path CSR, then the ordered carry fix-up
     hipEvent_t *te = timing_slot();
@@ -978,6 +984,7 @@ int Plan::trial(const std::vector<std::pair<int, int>> &forms, std::vector<float
   }
   timing = was_timing;
   cleanup();
+  ordered = false;  // nothing is left on the trial's stream
   if (st != SBLAS_OK) {
     if (st == SBLAS_ERR_HIP) set_error(SBLAS_ERR_HIP, "autotune: trial launch failed");
     return st;
@@ -1388,6 +1395,38 @@ int Plan::choose_csr(const std::vector<int> &h_rp) {
 bool Plan::uses_tiles(int k) const {
   return kernel == SBLAS_KERNEL_COO ||
          ((kernel == SBLAS_KERNEL_MERGE || kernel == SBLAS_KERNEL_CSR5) && k == 1);
+}
+
+// Whether a product writes memory of the plan that another would write too: tile
+// carries, sums over segments, an FP32 copy of x, partials of cut rows.
+bool Plan::shares_workspace(int k) const {
+  return uses_tiles(k) || variant == 6 || x32_rows || panel.x32 || !streams.empty() ||
+         has_merge(k);
+}
+
+// Such a product waits for the one before where that is on another stream.  The
+// event is recorded at the change of streams, so products that stay on one pay a
+// comparison; where the other stream is gone, so is its work.  A capture joins
+// no stream outside its graph: graphs of a plan are replayed one at a time.
+int Plan::follow_last(hipStream_t s) {
+  if (ordered && s == last_stream) return SBLAS_OK;
+  auto capturing = [](hipStream_t q) {
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(q, &c) == hipSuccess) return c != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+  };
+  if (capturing(s)) return SBLAS_OK;
+  if (ordered && !capturing(last_stream)) {
+    if (!last_event) SBLAS_HIP_TRY(hipEventCreateWithFlags(&last_event, hipEventDisableTiming));
+    if (hipEventRecord(last_event, last_stream) == hipSuccess)
+      SBLAS_HIP_TRY(hipStreamWaitEvent(s, last_event, 0));
+    else
+      (void)hipGetLastError();
+  }
+  ordered = true;
+  last_stream = s;
+  return SBLAS_OK;
 }
 
 bool Plan::has_merge(int k) const {

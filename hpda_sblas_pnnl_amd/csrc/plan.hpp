@@ -1,6 +1,7 @@
 // plan.hpp -- the engine's plan object behind the opaque sblas_plan handle.
 #pragma once
 
+#include <mutex>
 #include <vector>
 
 #include "internal.hpp"
@@ -136,6 +137,12 @@ struct Plan {
   bool rows_x32 = true;  // auto setting of narrow_x for row blocks (a trial may clear it)
   int launches = 0;
 
+  // products that keep sums in the plan follow one another (follow_last)
+  std::mutex order_mu;
+  bool ordered = false;               // last_stream holds such a product
+  hipStream_t last_stream = nullptr;
+  hipEvent_t last_event = nullptr;
+
   // kernel timing (measurement only)
   bool timing = false;
   std::vector<hipEvent_t> tev;   // pairs: [2i] before, [2i+1] after
@@ -165,6 +172,8 @@ struct Plan {
   // of four tiles for the CSR5-style kernel (its carries meet in LDS first)
   int carry_count() const { return kernel == SBLAS_KERNEL_CSR5 ? (tiles + 3) / 4 : tiles; }
   bool has_merge(int k) const;
+  bool shares_workspace(int k) const;
+  int follow_last(hipStream_t s);
   int setup_tiles();
   int setup_csr5(const std::vector<int> &h_rp);
   int narrow_x_asked() const;
