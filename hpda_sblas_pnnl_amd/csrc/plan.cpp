@@ -859,8 +859,9 @@ int Plan::setup_segments(int P) {
 // blocks.
 void Plan::setup_segment_vectors() {
   void *p[2] = {nullptr, nullptr};
-  const size_t bytes[2] = {sizeof(double) * kSegVectors * static_cast<size_t>(seg.M),
-                           sizeof(double) * kSegVectors * 2 * static_cast<size_t>(vsl.nblocks)};
+  const size_t most = four_over_segments() ? kSegVectors : 2;
+  const size_t bytes[2] = {sizeof(double) * most * static_cast<size_t>(seg.M),
+                           sizeof(double) * most * 2 * static_cast<size_t>(vsl.nblocks)};
   for (int i = 0; i < 2; i++)
     if (hipMalloc(&p[i], std::max<size_t>(bytes[i], 8)) != hipSuccess) {
       (void)hipGetLastError();
@@ -888,7 +889,7 @@ void Plan::setup_segment_vectors() {
 //     scale 22 (2.2) 687 / 631  917 / 884  1154 / 1153
 bool Plan::segment_vectors(int k) const {
   if (variant != 6 || !d_vsums || !streams.empty()) return false;
-  return k == 2 || (k == 4 && seg.M >= 3 * static_cast<int64_t>(m));
+  return k == 2 || (k == 4 && four_over_segments());
 }
 
 void Plan::drop_segments() {

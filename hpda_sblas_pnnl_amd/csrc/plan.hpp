@@ -108,7 +108,7 @@ struct Plan {
   int *d_vmrows = nullptr, *d_vmptr = nullptr, *d_vmslots = nullptr;
   int vgroups = 0;
   double *d_vpartials = nullptr;
-  double *d_vsums = nullptr;          // [seg.M][kSegVectors] of a multi-vector product, or nullptr
+  double *d_vsums = nullptr;          // [seg.M][2 or 4] of a multi-vector product, or nullptr
   double *d_vkpartials = nullptr;     // its partial slots
 
   // CSR5-style format (kernel 3)
@@ -191,6 +191,7 @@ struct Plan {
   void drop_segments();
   void setup_segment_vectors();
   bool segment_vectors(int k) const;
+  bool four_over_segments() const { return seg.M >= 3 * static_cast<int64_t>(m); }
   // times the given (kernel, variant) forms on the plan's own matrix; ms[i]
   // receives the median of form i.  Variants kLaneRows and kLaneSegments stand
   // for run_lanes.
