@@ -1068,8 +1068,16 @@ int Plan::build_sorted64(const std::vector<int> &h_rp, bool *chosen) {
   rule.few = 0;
   rule.chain = stats.max_row * panel_chain_us(rows) / (std::max<int64_t>(nnz, 1) / 6.05e5);
   panel = PanelFormat{};
-  return panel_build(val_type, rows, m, n, nnz, a0, a1, val, exec, h_rp.data(), false,
-                     rule, panel, chosen, nullptr, kPanelSorted);
+  const int st = panel_build(val_type, rows, m, n, nnz, a0, a1, val, exec, h_rp.data(), false,
+                             rule, panel, chosen, nullptr, kPanelSorted);
+  if (st != SBLAS_ERR_UNSUPPORTED && st != SBLAS_ERR_ALLOC) return st;
+  // no room: the forms that took the matrix before these panels
+  for (void *p : panel.buffers) (void)hipFree(p);
+  panel = PanelFormat{};
+  *chosen = false;
+  clear_error();
+  (void)hipGetLastError();
+  return SBLAS_OK;
 }
 
 // The plan's products run over its column panels from now on.
@@ -1096,17 +1104,7 @@ int Plan::use_panels(const std::vector<int> &h_rp) {
 // the results are then those of that copy.
 int Plan::band_panels(const std::vector<int> &h_rp, bool *chosen) {
   *chosen = false;
-  if (stats.max_row > 8192) return SBLAS_OK;
-  int st = build_sorted64(h_rp, chosen);
-  if (st == SBLAS_ERR_UNSUPPORTED || st == SBLAS_ERR_ALLOC) {
-    for (void *p : panel.buffers) (void)hipFree(p);
-    panel = PanelFormat{};
-    *chosen = false;
-    clear_error();
-    (void)hipGetLastError();
-    return SBLAS_OK;
-  }
-  return st;
+  return stats.max_row > 8192 ? static_cast<int>(SBLAS_OK) : build_sorted64(h_rp, chosen);
 }
 
 // Kernel choice and launch set-up for a CSR matrix whose row pointer is h_rp
@@ -1304,6 +1302,7 @@ int Plan::choose_csr(const std::vector<int> &h_rp) {
       st = ascend ? setup_segments(segments_for(n)) : static_cast<int>(SBLAS_ERR_UNSUPPORTED);
       if (st == SBLAS_ERR_ALLOC || st == SBLAS_ERR_UNSUPPORTED) {  // row blocks instead
         clear_error();
+        (void)hipGetLastError();  // launches to come must not find it
         drop_segments();
         return SBLAS_OK;
       }
@@ -1335,6 +1334,7 @@ int Plan::choose_csr(const std::vector<int> &h_rp) {
     st = setup_segments(segments_for(n));
     if (st == SBLAS_ERR_ALLOC || st == SBLAS_ERR_UNSUPPORTED) {
       clear_error();
+      (void)hipGetLastError();
       drop_segments();
     } else if (st != SBLAS_OK) {
       return st;
