@@ -237,7 +237,6 @@ int run(CallContext &c, int m, int n, int nnz, double alpha, const double *val,
     o_mslots = pack.add(mslots);
     const char *er = std::getenv("SBLAS_XCD_REMAP");
     L.items = 8;
-    L.subwave = 1;
     L.nblocks = static_cast<int>(rb.size());
     L.xcd_remap = !(er && *er) || std::atoi(er) != 0 ? 1 : 0;
     L.grid = L.xcd_remap ? (L.nblocks + 7) / 8 * 8 : L.nblocks;

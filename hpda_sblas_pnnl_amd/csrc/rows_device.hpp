@@ -1,6 +1,7 @@
 // rows_device.hpp -- what the row-block kernels share: the block order over the
-// XCDs (sblas_vector.hip, sblas_spmm.hip) and the row sums of an LDS-staged row
-// block (sblas_vector.hip, the column-sorted row blocks in sblas_sorted.hip).
+// XCDs (all of them, sblas_tiles.hip and sblas_csr5.hip) and the row sums of an
+// LDS-staged row block by groups of lanes (the column-sorted row blocks in
+// sblas_sorted.hip, sblas_lanes.hip).
 #pragma once
 
 #include "internal.hpp"

@@ -1,15 +1,16 @@
-// sblas_batch.hip -- many matrices of uneven sizes in one persistent launch.
+// sblas_batch.hip -- many matrices of uneven sizes in a few launches.
 //
 // Every matrix is cut into work items of the form its autotuner choice
 // names: row panels of the column-panel form (matrices whose rows draw x from
-// a wide window) or row blocks of the LDS-staged row form, and all items of
-// all matrices form one list in matrix order, cut into eight queues of equal
-// work, one per XCD.  A persistent grid sized to the resident workgroups
-// takes items from per-queue device counters (its own XCD's queue first,
-// then the others), so the launch balances itself across the GPU while
-// neighbouring items share that XCD's L2; an item's arithmetic (and so every sum) is
-// the same whichever workgroup runs it.  Each item carries its matrix's
-// parameters (arrays, value type, lanes per row), so matrices with different
+// a wide window) or row blocks of the LDS-staged row form, and the items of
+// each form make one list in matrix order, cut into eight queues of equal
+// work, one per XCD.  Row blocks run one item per workgroup.  Row panels run in a
+// persistent grid sized to the resident workgroups, which takes items from
+// per-queue device counters (its own XCD's queue first, then the others), so the
+// launch balances itself across the GPU while neighbouring items share that XCD's
+// L2; an item's arithmetic (and so every sum) is the same whichever workgroup runs
+// it.  (SBLAS_BATCH_FLAT gives either form the other kind of launch.)  Each item
+// carries its matrix's parameters (arrays, value type), so matrices with different
 // profiles share the launch.  Rows cut by an item's element window leave
 // partials that one merge launch combines in item order.
 #include "internal.hpp"

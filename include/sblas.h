@@ -15,7 +15,11 @@
  *   4. Matrix ingestion: the reference's COO sort / conversion helpers (on
  *      the device) and a Matrix Market reader.
  *
- * All functions are thread-safe.  Errors never exit the process: the
+ * All functions are thread-safe.  A plan runs one product at a time: products
+ * that keep sums in the plan (tiles, column segments, an FP32 copy of x, cut
+ * rows) follow one another also where they are called on different streams or
+ * threads; graphs captured from one plan must be replayed one at a time, and not
+ * beside its other products.  Errors never exit the process: the
  * functions return a status (or NaN timings for the spmv_ret entry points)
  * and sblas_last_error() holds the thread's last status.
  */
@@ -190,10 +194,10 @@ enum {
 };
 
 /* kernel AUTO: column panels (kernel 1) where the matrix's column structure
- * pays for them; otherwise row blocks or column-sorted row blocks (kernel 1)
- * or the CSR5-style kernel 3, whichever a timed trial on the matrix finds
- * fastest (matrices of at least 2^20 elements; smaller ones take row
- * blocks).  Trials are cached by row
+ * pays for them; otherwise row blocks, column-sorted row blocks, row blocks over
+ * column segments (kernel 1) or the CSR5-style kernel 3, whichever a timed trial
+ * on the matrix finds fastest (matrices of at least 2^20 elements; smaller ones
+ * take row blocks).  Trials are cached by row
  * profile; SBLAS_AUTOTUNE=0 turns them off.  sigma 0: the reference's rule
  * (include/anonymouslib_cuda.h:294-318) snapped to 8, 16 or 32.
  * chunks 0: SBLAS_CHUNKS when set, else one chunk per stream (one chunk for
@@ -205,7 +209,10 @@ typedef struct sblas_opts {
   int part_mode;   /* SBLAS_PART_*                                          */
   int nb;          /* v2 task size in nnz (part_mode V2)                    */
   int streams;     /* >1: one launch per chunk over this many streams       */
-  int subwave;     /* vector kernel lanes per row (0 = from row lengths)    */
+  int subwave;     /* lanes per row (0 = from row lengths) of the sub-wave  */
+                   /* form and of column-sorted row blocks; a power of two;  */
+                   /* checked for row blocks and segments, whose rows are    */
+                   /* summed by spans of elements whatever it says           */
   int sigma;       /* CSR5 nnz per lane per tile (0 = autotuned)            */
   int xcd_remap;   /* 1: contiguous row ranges per XCD; 0: off; -1: auto   */
   int variant;     /* kernel 1 form: 0 auto, 1 sub-wave per row, 2 row blocks */
@@ -219,14 +226,18 @@ typedef struct sblas_opts {
   int panel_rows;  /* column-panel form: rows per row panel (1..2048, or   */
                    /* 1..1536 in a batch; 0 auto)                           */
   int narrow_x;    /* FP32 / BF16 values, x in FP32: 0 auto (on for column  */
-                   /* panels, and for row blocks of >= 2^20 elements), 1    */
-                   /* off: x in FP64, each row summed in the host loop's    */
-                   /* order; 2 on: x staged or gathered from an FP32 copy   */
-                   /* written by each product (error within a few FP32      */
+                   /* panels that span several column panels, and for row   */
+                   /* blocks and segments of >= 2^20 elements where rows    */
+                   /* summed by groups of lanes are timed no slower than    */
+                   /* column-sorted blocks: info reports which), 1 off: x   */
+                   /* in FP64, in column panels each row summed in the host */
+                   /* loop's order; 2 on: x staged or gathered from an FP32 */
+                   /* copy written by each product (error within a few FP32 */
                    /* roundings per product); in a batch a narrow-x matrix  */
                    /* in column-panel form runs as a launch of its own      */
   int panel_layout;  /* column-panel form of a plan, layout inside a slice: */
-                     /* 0 auto (2 where x is staged in FP32, else 1), 1    */
+                     /* 0 auto (2 where x is staged in FP32, and with x in  */
+                     /* FP64 for rows of much the same length; else 1), 1  */
                      /* rows in order (one thread per row sums staged      */
                      /* products), 2 rows sorted by length in groups of 64 */
                      /* (one lane per row, padded to the group's longest); */
@@ -277,7 +288,10 @@ int sblas_plan_spmv(sblas_plan plan, double alpha, const double *d_x, double bet
 int sblas_plan_spmm(sblas_plan plan, int k, double alpha, const double *d_X,
                     double beta, double *d_Y, void *stream);
 typedef struct sblas_plan_info {
-  int format, val_type, kernel, chunks, subwave, sigma, xcd_remap, split_rows;
+  int format, val_type, kernel, chunks;
+  int subwave;       /* lanes per row (opts.subwave; of no effect in row    */
+                     /* blocks and segments)                                */
+  int sigma, xcd_remap, split_rows;
   int64_t m, n, nnz;
   int64_t workspace_bytes;
   double mean_row, cv_row;
@@ -297,7 +311,7 @@ typedef struct sblas_plan_info {
                      /* 2), CSR5-style (kernel 3), column-sorted row blocks  */
                      /* (kernel 1 variant 4); 0 without a trial              */
   int panel_layout;  /* column-panel form: 1 rows in order, 2 sorted groups */
-  int narrow_x;      /* column-panel form: 1 when x is staged in FP32       */
+  int narrow_x;      /* 1 when x is staged or gathered in FP32              */
   int64_t panel_elements; /* column-panel form: elements stored (padding    */
                           /* included)                                      */
   int segments;           /* variant 6: column segments                     */
@@ -324,11 +338,11 @@ int sblas_plan_kernel_times(sblas_plan plan, float *ms, int cap);
  * alive and unchanged while the batch exists.  A run is a launch of its own
  * for each large FP32 / BF16 matrix in column-panel form (on the caller's
  * stream, one after another), a persistent launch over the other matrices'
- * row panels and one over their row blocks (one work item per workgroup when
- * launches of their own run beside it; each on a stream forked from the
- * caller's and joined back; narrow row-block matrices of 2^20 elements or
- * more gather x from FP32 copies written by one launch ahead of them), then
- * one merge launch.  A batch runs one call at a time. */
+ * row panels and one over their row blocks (one work item per workgroup; each
+ * on a stream forked from the caller's and joined back; narrow row-block
+ * matrices of 2^20 elements or more gather x from FP32 copies written by one
+ * launch ahead of them, unless their rows are too uneven for the row panels that
+ * read x in FP64), then one merge launch.  A batch runs one call at a time. */
 typedef struct sblas_batch_item {
   int m, n;
   int64_t nnz;
@@ -346,7 +360,7 @@ typedef struct sblas_batch_item {
 /* What the autotuner picked for one matrix. */
 typedef struct sblas_batch_choice {
   int kernel;      /* SBLAS_KERNEL_VECTOR (kernel 1)                        */
-  int subwave;     /* lanes per row                                          */
+  int subwave;     /* lanes per row of multi-vector items                    */
   int items;       /* elements per thread of a row block                     */
   int chunks;      /* nnz chunks the row blocks are cut from                 */
   int row_blocks;  /* work items of this matrix (row blocks or row panels)   */
