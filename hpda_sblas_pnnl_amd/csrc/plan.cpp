@@ -222,8 +222,6 @@ int upload(Plan &p, T **dst, const std::vector<T> &src) {
 
 }  // namespace
 
-namespace {
-
 // Small host arrays uploaded together: one allocation and one transfer (a
 // synchronous transfer of its own costs each about 15 us).
 class Uploads {
@@ -251,8 +249,6 @@ class Uploads {
   std::vector<char> bytes_;
   std::vector<std::pair<void **, size_t>> places_;
 };
-
-}  // namespace
 
 int Plan::build_csr_chunks(const int *h_rp) {
   const int C = chunks;
@@ -415,15 +411,18 @@ int Plan::setup_stream(const int *h_rp) {
   up.add(&d_bmrows, mrows);
   up.add(&d_bmptr, mptr);
   up.add(&d_bmslots, mslots);
+  const size_t shorter = setup_short_blocks(h_rp, up);
   if ((st = up.send(*this)) != SBLAS_OK) return st;
   // 2 slots per block, max_k values per slot (multi-RHS blocks use the same list)
+  const size_t slots = 2 * static_cast<size_t>(max_k);
   d_bpartials = static_cast<double *>(
-      dev_alloc(sizeof(double) * 2 * max_k * std::max<size_t>(rblocks.size(), 1)));
+      dev_alloc(sizeof(double) * slots * (std::max<size_t>(rblocks.size(), 1) + shorter)));
   if (!d_bpartials) {
     set_error(SBLAS_ERR_ALLOC, "plan: partials allocation failed");
     return SBLAS_ERR_ALLOC;
   }
-  return setup_short_blocks(h_rp);
+  d_kpartials = d_bpartials + slots * std::max<size_t>(rblocks.size(), 1);
+  return SBLAS_OK;
 }
 
 // Row blocks of 512 elements for products of 8 or 16 vectors over matrices of
@@ -434,11 +433,12 @@ int Plan::setup_stream(const int *h_rp) {
 // 15.6; 10,000 rows of 7 (35) 9.5 / 15.4 -> 4.7 / 6.0; 100,000 rows of 10 (491)
 // 10.7 / 14.4 -> 9.1 / 12.1; above, equal or slower (power law, 60,000 rows, 516
 // blocks: 15.0 / 20.0 -> 17.1 / 21.5; R-MAT 300,000 rows 63 / 83 -> 76 / 93).
-int Plan::setup_short_blocks(const int *h_rp) {
+// Their lists go up with `up`; returns their number (0: none).
+size_t Plan::setup_short_blocks(const int *h_rp, Uploads &up) {
   slk = StreamLaunch{};
   int cus = 256;
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
-  if (opts.items > 0 || sl.nblocks > 2 * std::max(cus, 1)) return SBLAS_OK;
+  if (opts.items > 0 || sl.nblocks > 2 * std::max(cus, 1)) return 0;
   const int items = 2;
   const std::vector<RowBlock> kb = build_row_blocks(exec, h_rp, kStreamBlock * items);
   std::vector<ExecChunk> as_chunks;
@@ -447,24 +447,15 @@ int Plan::setup_short_blocks(const int *h_rp) {
   std::vector<int> mrows, mptr, mslots;
   merge_lists(as_chunks, h_rp, mrows, mptr, mslots);
   kgroups = static_cast<int>(mrows.size());
-  int st;
-  Uploads up;
   up.add(&d_kblocks, kb);
   up.add(&d_kmrows, mrows);
   up.add(&d_kmptr, mptr);
   up.add(&d_kmslots, mslots);
-  if ((st = up.send(*this)) != SBLAS_OK) return st;
-  d_kpartials = static_cast<double *>(
-      dev_alloc(sizeof(double) * 2 * max_k * std::max<size_t>(kb.size(), 1)));
-  if (!d_kpartials) {
-    set_error(SBLAS_ERR_ALLOC, "plan: partials allocation failed");
-    return SBLAS_ERR_ALLOC;
-  }
   slk = sl;
   slk.items = items;
   slk.nblocks = static_cast<int>(kb.size());
   slk.grid = slk.xcd_remap ? ((slk.nblocks + 7) / 8) * 8 : slk.nblocks;
-  return SBLAS_OK;
+  return kb.size();
 }
 
 hipEvent_t *Plan::timing_slot() {

@@ -36,6 +36,8 @@ VectorLaunch vector_shape(const std::vector<ExecChunk> &ex, double mean, int sub
 void merge_lists(const std::vector<ExecChunk> &ex, const int *rp, std::vector<int> &rows,
                  std::vector<int> &ptr, std::vector<int> &slots);
 
+class Uploads;  // small host arrays sent to the device together (plan.cpp)
+
 struct Plan {
   int format = SBLAS_FMT_CSR;
   int val_type = SBLAS_VAL_F64;
@@ -153,7 +155,7 @@ struct Plan {
   int build_csr_chunks(const int *h_rp);
   int setup_vector(const int *h_rp);
   int setup_stream(const int *h_rp);
-  int setup_short_blocks(const int *h_rp);
+  size_t setup_short_blocks(const int *h_rp, Uploads &up);
   // With 8 vectors they must not bring a merge launch that the long blocks do
   // without, unless those are fewer still (power law, 20,000 rows, 171 blocks:
   // 9.4 us with long blocks, 9.7 with short ones).

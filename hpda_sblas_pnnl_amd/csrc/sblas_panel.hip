@@ -168,22 +168,45 @@ __global__ void k_panel_range(int npanels, PanelInfo *__restrict__ info,
 
 // *diff = columns that descend from one element to the next, less those that
 // do so from one row's last element to the next row's first: 0 when every
-// row's columns ascend.
+// row's columns ascend.  Bound by HBM reads of the columns: a thread's
+// kOrderItems loads are in flight together, and a workgroup adds to *diff once
+// (56 M columns: 231 us with one load after another and an addition a wave,
+// ORDER_NOW us).
+constexpr int kOrderItems = 8;
+constexpr int kOrderBlocks = 2048;  // workgroups at most
 __global__ __launch_bounds__(256) void k_column_order(int m, int64_t nnz,
                                                       const int *__restrict__ rp,
                                                       const int *__restrict__ col,
                                                       unsigned long long *__restrict__ diff) {
   const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
   const int64_t first = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  long long d = 0;
-  for (int64_t j = first + 1; j < nnz; j += stride) d += col[j] < col[j - 1] ? 1 : 0;
+  __shared__ int sums[4];
+  int d = 0;  // at most the elements and rows of one thread
+  for (int64_t base = static_cast<int64_t>(blockIdx.x) * 256 * kOrderItems; base < nnz;
+       base += stride * kOrderItems) {
+    int c[kOrderItems], before[kOrderItems];
+#pragma unroll
+    for (int k = 0; k < kOrderItems; k++) {
+      const int64_t j = min<int64_t>(base + k * 256 + threadIdx.x, nnz - 1);
+      c[k] = col[j];
+      before[k] = col[j > 0 ? j - 1 : 0];
+    }
+#pragma unroll
+    for (int k = 0; k < kOrderItems; k++)
+      if (base + k * 256 + threadIdx.x < nnz) d += c[k] < before[k] ? 1 : 0;
+  }
   for (int64_t r = first; r < m; r += stride) {
     const int b = rp[r];
     if (b > 0 && rp[r + 1] > b) d -= col[b] < col[b - 1] ? 1 : 0;
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) d += __shfl_xor(d, off, 64);
-  if ((threadIdx.x & 63) == 0 && d != 0) atomicAdd(diff, static_cast<unsigned long long>(d));
+  if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = d;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const long long all = static_cast<long long>(sums[0]) + sums[1] + sums[2] + sums[3];
+    if (all != 0) atomicAdd(diff, static_cast<unsigned long long>(all));
+  }
 }
 
 // Element-parallel passes over one row panel's element window: one
@@ -376,7 +399,8 @@ int columns_ascend(int m, int64_t nnz, const int *rp, const int *col, hipStream_
   SBLAS_HIP_TRY(hipMalloc(&diff, sizeof(h)));
   hipError_t e = hipMemcpyAsync(diff, &h, sizeof(h), hipMemcpyHostToDevice, s);
   if (e == hipSuccess) {
-    const int64_t blocks = std::min<int64_t>((nnz + 1023) / 1024, 4096);
+    const int64_t blocks =
+        std::min<int64_t>((nnz + 256 * kOrderItems - 1) / (256 * kOrderItems), kOrderBlocks);
     hipLaunchKernelGGL(k_column_order, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, m, nnz,
                        rp, col, diff);
     e = hipGetLastError();
