@@ -171,7 +171,7 @@ __global__ void k_panel_range(int npanels, PanelInfo *__restrict__ info,
 // row's columns ascend.  Bound by HBM reads of the columns: a thread's
 // kOrderItems loads are in flight together, and a workgroup adds to *diff once
 // (56 M columns: 231 us with one load after another and an addition a wave,
-// ORDER_NOW us).
+// 53 us).
 constexpr int kOrderItems = 8;
 constexpr int kOrderBlocks = 2048;  // workgroups at most
 __global__ __launch_bounds__(256) void k_column_order(int m, int64_t nnz,
@@ -338,14 +338,17 @@ __global__ void k_panel_slice_scan(int nslices, int R, const uint32_t *__restric
 // t*RPT .. t*RPT+RPT-1 of the order.  perm[slice * R + i] = the row at place
 // i, rank[slice * R + row] = its place, goff[slice * (G + 1) + g] = 64 times
 // the summed lengths of groups before g (a group's length is its first
-// row's count), snnz[slice] = the slice's stored elements.
+// row's count), snnz[slice] = the slice's stored elements.  A count passes
+// kPanelCols only where a row repeats columns; past 13 bits the slice is sorted
+// on the whole count, and offsets past 31 bits are flagged.
 template <int RPT>
 __global__ __launch_bounds__(256) void k_sorted_slice_order(int nslices, int R,
                                                             const uint32_t *__restrict__ cnt,
                                                             uint16_t *__restrict__ perm,
                                                             uint16_t *__restrict__ rank,
                                                             uint32_t *__restrict__ goff,
-                                                            int64_t *__restrict__ snnz) {
+                                                            int64_t *__restrict__ snnz,
+                                                            int *__restrict__ overflow) {
   typedef hipcub::BlockRadixSort<uint32_t, 256, RPT, uint16_t> Sort;
   __shared__ typename Sort::TempStorage tmp;
   __shared__ uint32_t glen[kPanelRowsMax / 64];
@@ -361,8 +364,13 @@ __global__ __launch_bounds__(256) void k_sorted_slice_order(int nslices, int R,
     key[j] = i < R ? cnt[static_cast<int64_t>(s) * R + i] : 0u;
     row[j] = static_cast<uint16_t>(i);
   }
-  // counts are at most kPanelCols (13 bits)
-  Sort(tmp).SortDescending(key, row, 0, 13);
+  bool wide = false;
+#pragma unroll
+  for (int j = 0; j < RPT; j++) wide |= key[j] >> 13 != 0;
+  if (__syncthreads_or(wide))
+    Sort(tmp).SortDescending(key, row, 0, 32);
+  else
+    Sort(tmp).SortDescending(key, row, 0, 13);
 #pragma unroll
   for (int j = 0; j < RPT; j++) {
     const int i = t * RPT + j;
@@ -374,12 +382,13 @@ __global__ __launch_bounds__(256) void k_sorted_slice_order(int nslices, int R,
   }
   __syncthreads();
   if (t == 0) {
-    uint32_t off = 0;
+    int64_t off = 0;
     for (int g = 0; g < G; g++) {
-      goff[static_cast<int64_t>(s) * (G + 1) + g] = off;
-      off += 64u * glen[g];
+      goff[static_cast<int64_t>(s) * (G + 1) + g] = static_cast<uint32_t>(off);
+      off += 64 * static_cast<int64_t>(glen[g]);
     }
-    goff[static_cast<int64_t>(s) * (G + 1) + G] = off;
+    goff[static_cast<int64_t>(s) * (G + 1) + G] = static_cast<uint32_t>(off);
+    if (off > 0x7FFFFFFF) overflow[0] = 1;
     snnz[s] = off;  // a multiple of 64: slices start aligned
   }
 }
@@ -565,7 +574,7 @@ int panel_build(int val_type, int rows, int m, int n, int64_t nnz, const int *rp
 #define SBLAS_ORDER_CASE(RPT)                                                                 \
   case RPT:                                                                                   \
     hipLaunchKernelGGL(k_sorted_slice_order<RPT>, dim3(f.nslices), dim3(256), 0, s, f.nslices, \
-                       R, cnt, f.perm, rank, f.goff, snnz);                                   \
+                       R, cnt, f.perm, rank, f.goff, snnz, overflow);                         \
     break;
     switch (f.rpt) {
       SBLAS_ORDER_CASE(1)
@@ -593,6 +602,10 @@ int panel_build(int val_type, int rows, int m, int n, int64_t nnz, const int *rp
   int h_over = 0;
   SBLAS_HIP_TRY(hipMemcpyAsync(&h_over, overflow, sizeof(int), hipMemcpyDeviceToHost, s));
   SBLAS_HIP_TRY(hipStreamSynchronize(s));
+  if (h_over && sorted) {
+    set_error(SBLAS_ERR_UNSUPPORTED, "panel format: a slice's padded elements pass 31 bits");
+    return SBLAS_ERR_UNSUPPORTED;
+  }
   if (!h_over && !sorted) {
     // every slice fits 16-bit offsets: keep the narrow copy only
     // two entries of slack: the kernel stages a slice's offsets as whole
